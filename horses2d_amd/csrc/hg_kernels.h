@@ -45,46 +45,158 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
     return x * per + (x < rem ? x : rem) + q;
 }
 
+// LDS layout of an element's nodes: node (i, j) is entry i + RS j of ES entries per element, an
+// entry being 16 bytes of each plane (Quads below).  The pads spread the rows (P = 4 and 8, whose
+// rows of 64 and 128 B otherwise share banks) or the elements of a tile (P = 3, 6, 7) over the
+// banks.  The row and column reads of a wide tile's FP64 contraction, and its trace reads, timed
+// alone (one 32-byte entry per node without pads -> this layout): P = 3 29 -> 16 and 23 -> 16 us,
+// P = 4 38 -> 25 and 37 -> 21, P = 5 38 -> 30 and 31 -> 23, P = 6 53 -> 38 and 28 -> 20,
+// P = 7 45 -> 40 and 29 -> 23, P = 8 92 -> 45 and 72 -> 22, P = 9 71 -> 53 and 31 -> 23; pads at
+// the other orders gain nothing.
+template <int P>
+struct Layout {
+    static constexpr int RS = P + ((P == 4 || P == 8) ? 1 : 0);
+    static constexpr int ES = P * RS + ((P == 3 || P == 6) ? 3 : P == 7 ? 7 : 0);
+    // entry of node n (= i + P j) of the tile's element s
+    __device__ static constexpr int at(int s, int n) { return s * ES + n + (RS - P) * (n / P); }
+};
+
 template <int P, int EPB_>
 struct Tile {
     static constexpr int PP = P * P;
     static constexpr int EPB = EPB_;
     static constexpr int NF = EPB * 4 * P;
     static constexpr int NN = EPB * PP;
+    static constexpr int NL = EPB * Layout<P>::ES;   // entries of a node array in LDS
     static constexpr int TPB = (((NN > NF ? NN : NF) + 63) / 64) * 64;
 };
 
+// Arrays of NL four-value entries in LDS.  FP64: two planes of 16-byte halves (entry x of plane h
+// holds values 2 h, 2 h + 1), so that neighbouring entries are 16 bytes apart for every ds_read_b128
+// instead of 32, where half of the banks were visited twice; FP32: one plane of float4.
+template <typename R, int NL>
+struct Quads {
+    static constexpr int SIZE = 4 * NL;   // values of R
+    __device__ static __forceinline__ void get(const R *A, int x, R *v) {
+        if constexpr (sizeof(R) == 8) {
+            const double2 a = *(const double2 *)(A + 2 * x), b = *(const double2 *)(A + 2 * NL + 2 * x);
+            v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
+        } else {
+            const float4 a = *(const float4 *)(A + 4 * x);
+            v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+        }
+    }
+    __device__ static __forceinline__ void put(R *A, int x, const R *v) {
+        if constexpr (sizeof(R) == 8) {
+            *(double2 *)(A + 2 * x) = make_double2(v[0], v[1]);
+            *(double2 *)(A + 2 * NL + 2 * x) = make_double2(v[2], v[3]);
+        } else {
+            *(float4 *)(A + 4 * x) = make_float4(v[0], v[1], v[2], v[3]);
+        }
+    }
+    // values 2 h and 2 h + 1 of entry x
+    __device__ static __forceinline__ void get_half(const R *A, int x, int h, R &a, R &b) {
+        if constexpr (sizeof(R) == 8) {
+            const double2 v = *(const double2 *)(A + 2 * NL * h + 2 * x);
+            a = v.x; b = v.y;
+        } else {
+            const float2 v = *(const float2 *)(A + 4 * x + 2 * h);
+            a = v.x; b = v.y;
+        }
+    }
+};
+
+// Trace of a face from the staged element state (DGSpatialDiscretizationMethods.f90:1520-1574):
+// X is an array of NL entries (Quads), x0 the element's first.  Accumulated in FP64 with explicit
+// fma in l order so that every kernel that forms a trace (prolongation, stage epilogue) produces
+// the same bits; A = T accumulates in the tile's own type (the FP32 form's gradient traces, which
+// only the kernel that forms them ever evaluates).
+template <int P, int NL, typename T, typename A>
+__device__ __forceinline__ void face_trace(const T *X, int x0, const A *sLb, int f, int k, A *out) {
+    const A *lb = (f == 0 || f == 3) ? sLb : sLb + P;
+    // nodes (k, l) of a horizontal face or (l, k) of a vertical one: a base and a stride, so
+    // the loop body has no face-dependent branch
+    constexpr int RS = Layout<P>::RS;
+    const bool horiz = (f == 0 || f == 2);
+    const int base = x0 + (horiz ? k : RS * k), step = horiz ? RS : 1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) out[c] = A(0);
+    // a rolled loop keeps one node's values live (unrolled, all P nodes are loaded up front)
+#pragma unroll 1
+    for (int l = 0; l < P; ++l) {
+        T v[4];
+        Quads<T, NL>::get(X, base + step * l, v);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) out[c] = fma((A)v[c], lb[l], out[c]);
+    }
+}
+
+// The same for an eight-value array (two Quads arrays one after the other): one pass over the nodes.
+template <int P, int NL, typename T, typename A>
+__device__ __forceinline__ void face_trace8(const T *X, int x0, const A *sLb, int f, int k, A *out) {
+    const A *lb = (f == 0 || f == 3) ? sLb : sLb + P;
+    constexpr int RS = Layout<P>::RS;
+    const bool horiz = (f == 0 || f == 2);
+    const int base = x0 + (horiz ? k : RS * k), step = horiz ? RS : 1;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) out[c] = A(0);
+#pragma unroll 1
+    for (int l = 0; l < P; ++l) {
+        T v[8];
+        Quads<T, NL>::get(X, base + step * l, v);
+        Quads<T, NL>::get(X + Quads<T, NL>::SIZE, base + step * l, v + 4);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) out[c] = fma((A)v[c], lb[l], out[c]);
+    }
+}
+
 // Tile choices: 0 = widest tile within one wavefront, 1 = widest within four wavefronts whose
-// Euler FP64 LDS tile (state, two contravariant fluxes, face fluxes: 96 P^2 + 128 P bytes per
-// element) stays within 31 KB, so that five workgroups fit a CU's LDS (this caps P = 4 at 15
-// elements instead of 16; the batched kernels' LDS is the largest tile over all orders).
+// Euler FP64 LDS tile (state, two contravariant fluxes, face fluxes: 96 ES + 128 P bytes per
+// element) stays within 31 KB, so that five workgroups fit a CU's LDS (the batched kernels' LDS
+// is the largest tile over all orders).  P = 4: 12 elements, three full wavefronts, where 13 fit.
 template <int P>
 struct Tiles {
     static constexpr int a64 = 64 / (P * P), b64 = 64 / (4 * P);
     static constexpr int a256 = 256 / (P * P), b256 = 256 / (4 * P);
-    static constexpr int lds_cap = (31 * 1024) / (96 * P * P + 128 * P);
+    static constexpr int lds_fit = (31 * 1024) / (96 * Layout<P>::ES + 128 * P);
+    static constexpr int lds_cap = P == 4 ? 12 : lds_fit;
     static constexpr int small = (a64 < b64 ? a64 : b64) > 0 ? (a64 < b64 ? a64 : b64) : 1;
     static constexpr int wide = (a256 < b256 ? a256 : b256) > 0 ? (a256 < b256 ? a256 : b256) : 1;
     static constexpr int large = (wide < lds_cap ? wide : lds_cap) > 0 ? (wide < lds_cap ? wide : lds_cap) : 1;
 };
 
+// Stages an element tile's state from HBM into LDS: FP64 (KEEP64), plus the compute-type copy
+// (energy slot shifted) that the gradient contractions read when the compute type is FP32.
+template <int P, int NL, typename R, bool COPY, bool KEEP64 = true>
+__device__ __forceinline__ void load_tile(const StageArgs &a, const int64_t nb0, const int ne, double *sQ, R *sQf,
+                                          const int t, const int TPB) {
+    constexpr int PP = P * P;
+    const double2 *src = (const double2 *)(a.Q + nb0 * 4);
+    for (int x = t; x < ne * PP * 2; x += TPB) {
+        // pairs (0, 1) and (2, 3) of a node: the odd pair holds the energy
+        const double2 v = src[x];
+        const int h = x & 1, e = Layout<P>::at((x >> 1) / PP, (x >> 1) % PP);
+        if constexpr (KEEP64) *(double2 *)(sQ + 2 * NL * h + 2 * e) = v;
+        if constexpr (COPY)
+            *(float2 *)(sQf + 4 * e + 2 * h) = make_float2((float)v.x, (float)(h ? slot_energy<R>(a.ph, v.y) : v.y));
+    }
+}
+
 // ------------------------------------------------------------------ prolongation
 template <int P, int EPB, typename TR>
 __global__ __launch_bounds__((Tile<P, EPB>::TPB)) void k_prolong(StageArgs a) {
     using T = Tile<P, EPB>;
-    __shared__ double sQ[T::NN * 4];
+    __shared__ __align__(16) double sQ[T::NL * 4];
     __shared__ double sLb[2 * P];
     const int t = threadIdx.x, e0 = blockIdx.x * EPB;
     if (t < 2 * P) sLb[t] = a.lb[t];
-    const int64_t base = (int64_t)e0 * T::PP * 4;
-    const int nval = min(EPB, a.K - e0) * T::PP * 4;
-    for (int x = t; x < nval; x += T::TPB) sQ[x] = a.Q[base + x];
+    load_tile<P, T::NL, double, false>(a, (int64_t)e0 * T::PP, min(EPB, a.K - e0), sQ, (double *)nullptr, t, T::TPB);
     __syncthreads();
     if (t < T::NF) {
         const int s = t / (4 * P), f = (t / P) % 4, k = t % P, e = e0 + s;
         if (e < a.K) {
             double tq[4];
-            face_trace<P, 4, 4>(sQ + s * T::PP * 4, sLb, f, k, tq);
+            face_trace<P, T::NL>(sQ, s * Layout<P>::ES, sLb, f, k, tq);
             tq[3] = slot_energy<TR>(a.ph, tq[3]);
             TR *o = (TR *)a.tr_out + ((int64_t)(e * 4 + f) * P + k) * 4;
 #pragma unroll
@@ -150,46 +262,52 @@ __device__ __forceinline__ void br1_face_flux(const StageArgs &a, const Phys<R> 
 
 // BR1 gradient at node (i, j): ( -Vector_StdVolumeGreen(Q) + sum_faces Vector_StdFace(uStar) ) / jac
 // (DGViscous_BR1.f90:48-111, DGWeakIntegrals.f90:503-622), faces lifted in edge-id order.
-// q: element state in the compute type [n*4] (energy slot shifted in the FP32 form),
-// Ja: element metric [n*4], Fu: element uStar fluxes [(f*P + k)*6] (see br1_face_flux).
+// q: the tile's state in the compute type (Quads; energy slot shifted in the FP32 form), Ja: its
+// metric (Quads: Ja11, Ja21, Ja12, Ja22), x0 the element's first entry in both, Fu: element uStar
+// fluxes [(f*P + k)*6] (see br1_face_flux), sHat: hatD transposed (hatD(i, l) at [l*P + i]).
 // ROLLED keeps the two l loops rolled (one node's values live; the stage kernel, where the
 // registers bound occupancy); the sums are the same either way.
 // Faces whose bit 8 + f is set in ord are curved p-non-conforming or subdivided edges, whose
 // lift terms come per direction from the mortar kernel (uStar dS n projected direction by
 // direction): the face lane stores the x terms with the "normal" (1, 0), and mortar_y_lift adds
 // the y terms afterwards.
-template <int P, typename R, int QS = 4, int JS = 4, bool ROLLED = false>
-__device__ __forceinline__ void br1_node_gradient(const R *q, const R *Ja, const R *sHat, const R *Fu, const R *sLbw,
-                                                  int ord, int i, int j, R ijac, R *dq) {
+template <int P, int NL, typename R, bool ROLLED = false>
+__device__ __forceinline__ void br1_node_gradient(const R *q, const R *Ja, int x0, const R *sHat, const R *Fu,
+                                                  const R *sLbw, int ord, int i, int j, R ijac, R *dq) {
     // Every accumulator receives its xi terms (l = 0..P-1) then its eta terms; each state value
     // is read once and used for both directions, and the metric-weighted derivative entry
     // Ja * hatD is formed once per node for all four variables.
-    constexpr int UNROLL = ROLLED ? 1 : P;
+    constexpr int UNROLL = ROLLED ? 1 : P, RS = Layout<P>::RS;
+    using V = Quads<R, NL>;
     R acc[8];
 #pragma unroll
     for (int c = 0; c < 8; ++c) acc[c] = R(0);
 #pragma unroll UNROLL
     for (int l = 0; l < P; ++l) {
-        const int m = l + P * j;
-        const R h = sHat[i * P + l];
-        const R w0 = Ja[m * JS + 0] * h, w2 = Ja[m * JS + 2] * h;
+        const int m = x0 + l + RS * j;
+        const R h = sHat[l * P + i];
+        R j11, j21, v[4];
+        V::get_half(Ja, m, 0, j11, j21);
+        V::get(q, m, v);
+        const R w0 = j11 * h, w2 = j21 * h;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const R v = q[m * QS + c];
-            acc[c] += v * w0;
-            acc[4 + c] += v * w2;
+            acc[c] += v[c] * w0;
+            acc[4 + c] += v[c] * w2;
         }
     }
 #pragma unroll UNROLL
     for (int l = 0; l < P; ++l) {
-        const int m = i + P * l;
-        const R h = sHat[j * P + l];
-        const R w1 = Ja[m * JS + 1] * h, w3 = Ja[m * JS + 3] * h;
+        const int m = x0 + i + RS * l;
+        const R h = sHat[l * P + j];
+        R j12, j22, v[4];
+        V::get_half(Ja, m, 1, j12, j22);
+        V::get(q, m, v);
+        const R w1 = j12 * h, w3 = j22 * h;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const R v = q[m * QS + c];
-            acc[c] += v * w1;
-            acc[4 + c] += v * w3;
+            acc[c] += v[c] * w1;
+            acc[4 + c] += v[c] * w3;
         }
     }
 #pragma unroll
@@ -229,15 +347,18 @@ __device__ __forceinline__ void mortar_y_lift(const double *mu8, const R *sLbw, 
 }
 
 // Interior (broken) gradient of the IP method (QuadElement_QuadProcedures.incf:42-88); q as above.
-template <int P, typename R, int QS = 4>
-__device__ __forceinline__ void ip_node_gradient(const R *q, const R *sD, int i, int j, R j11, R j12, R j21, R j22,
-                                                 R ijac, R *dq) {
+// sD: D transposed (D(i, l) at [l*P + i]).
+template <int P, int NL, typename R>
+__device__ __forceinline__ void ip_node_gradient(const R *q, int x0, const R *sD, int i, int j, R j11, R j12, R j21,
+                                                 R j22, R ijac, R *dq) {
     // l outermost (each accumulator still sums l = 0..P-1 in order): one node's values live
     R dxi[4] = {R(0), R(0), R(0), R(0)}, deta[4] = {R(0), R(0), R(0), R(0)};
 #pragma unroll 1
     for (int l = 0; l < P; ++l) {
-        const R di = sD[i * P + l], dj = sD[j * P + l];
-        const R *qx = q + (l + P * j) * QS, *qy = q + (i + P * l) * QS;
+        const R di = sD[l * P + i], dj = sD[l * P + j];
+        R qx[4], qy[4];
+        Quads<R, NL>::get(q, x0 + l + Layout<P>::RS * j, qx);
+        Quads<R, NL>::get(q, x0 + i + Layout<P>::RS * l, qy);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             dxi[c] += di * qx[c];
@@ -248,24 +369,6 @@ __device__ __forceinline__ void ip_node_gradient(const R *q, const R *sD, int i,
     for (int c = 0; c < 4; ++c) {
         dq[c] = (dxi[c] * j11 + deta[c] * j12) * ijac;
         dq[4 + c] = (dxi[c] * j21 + deta[c] * j22) * ijac;
-    }
-}
-
-// Stages an element tile's state from HBM into LDS: FP64 always, plus the compute-type copy
-// (energy slot shifted) that the gradient contractions read when the compute type is FP32.
-// The FP64 tile has a node stride of QS doubles (4, or 6 in the gradient kernel).
-template <typename R, bool COPY, bool KEEP64 = true, int QS = 4>
-__device__ __forceinline__ void load_tile(const StageArgs &a, const int64_t nb0, const int ne, const int PP, double *sQ,
-                                          R *sQf, const int t, const int TPB) {
-    const double2 *src = (const double2 *)(a.Q + nb0 * 4);
-    double2 *dst = (double2 *)sQ;
-    for (int x = t; x < ne * PP * 2; x += TPB) {
-        const double2 v = src[x];
-        if constexpr (KEEP64) dst[(x >> 1) * (QS / 2) + (x & 1)] = v;
-        if constexpr (COPY) {
-            // pairs (0,1) and (2,3) of a node: the odd pair holds the energy
-            ((float2 *)sQf)[x] = make_float2((float)v.x, (float)((x & 1) ? slot_energy<R>(a.ph, v.y) : v.y));
-        }
     }
 }
 
@@ -335,35 +438,20 @@ __device__ __forceinline__ void stored_trace(const StageArgs &a, int fe, int ff,
     for (int c = 0; c < 4; ++c) qs[c] = (R)o[c];
 }
 
-// Own Q trace of a face node from the LDS tile, in the compute type, rounded like the stored
-// traces the neighbour reads.
-template <int P, typename R, typename TR>
-__device__ __forceinline__ void own_trace(const StageArgs &a, const double *sQe, const double *sLb, int ff, int fk,
-                                          R *qs) {
-    double tq[4];
-    face_trace<P, 4, 4>(sQe, sLb, ff, fk, tq);
-    tq[3] = slot_energy<TR>(a.ph, tq[3]);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) qs[c] = (R)(TR)tq[c];
-}
-
 // This side's viscous flux at a face node from its Q trace qs and the element's nodal gradient
-// tile (node stride DS), times mu, stored in the VT layout (ViscousFluxes.f90:39-80, adiabatic
+// tile (two Quads arrays, x0 the element's first entry), times mu, stored in the VT layout (ViscousFluxes.f90:39-80, adiabatic
 // walls :279-318).  The gradient trace is accumulated in FP64 in the FP64 form and in FP32 in
 // the FP32 form (lbR: lb in the compute type).
 // mdq: where a p-non-conforming face keeps its gradient trace for the mortar kernel (or null).
-template <int P, int DS, typename R, typename TR>
+template <int P, int NL, typename R, typename TR>
 __device__ __forceinline__ void viscous_face_trace(const StageArgs &a, const Phys<R> &ph, int flags, const R *qs,
-                                                   const R *sDQe, const double *sLb, const R *lbR, int ff, int fk,
-                                                   TR *o, R muf, double *mdq = nullptr) {
+                                                   const R *sDQ, int x0, const double *sLb, const R *lbR, int ff,
+                                                   int fk, TR *o, R muf, double *mdq = nullptr) {
     R ds[8], fv[4], gv[4];
     if constexpr (sizeof(R) == 4) {
-        face_trace_r<P, DS, 8>(sDQe, lbR, ff, fk, ds);
+        face_trace8<P, NL>(sDQ, x0, lbR, ff, fk, ds);
     } else {
-        double tg[8];
-        face_trace<P, DS, 8>(sDQe, sLb, ff, fk, tg);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) ds[c] = (R)(TR)tg[c];
+        face_trace8<P, NL>(sDQ, x0, sLb, ff, fk, ds);
     }
     if (mdq) {
 #pragma unroll
@@ -380,31 +468,19 @@ __device__ __forceinline__ void viscous_face_trace(const StageArgs &a, const Phy
 // them and the Q traces, this side's viscous flux at every face node, which both elements of
 // the face read in their stage kernels.  The gradient at the nodes is not stored: each stage
 // kernel recomputes it for its own element.
-// Node strides (in elements of the tile's type) of the gradient kernel's LDS tiles, chosen so
-// that the P nodes of a row or a column of an element fall in distinct LDS banks for 16-byte
-// reads: FP64 state and metric 48 B, FP64 gradient 80 B; the FP32 state copy and metric
-// (16 B per node) need no padding, the FP32 gradient is padded to 48 B.
-template <typename R>
-struct GradStrides {
-    static constexpr int QS = sizeof(R) == 8 ? 6 : 4;    // state (FP64 tile or FP32 copy)
-    static constexpr int JS = sizeof(R) == 8 ? 6 : 4;    // metric
-    static constexpr int DS = sizeof(R) == 8 ? 10 : 12;  // gradient
-};
-
 template <int P, int EPB, bool BR1, typename R>
 struct GradSmem {
     using T = Tile<P, EPB>;
-    using ST = GradStrides<R>;
     struct Inputs {
-        alignas(16) double sQ[sizeof(R) == 4 ? 2 : T::NN * ST::QS];   // FP64 form: the state
-        alignas(16) R sQf[sizeof(R) == 4 ? T::NN * ST::QS : 1];        // FP32 form: the compute-type state
-        alignas(16) R sJa[BR1 ? T::NN * ST::JS : 1];
+        alignas(16) double sQ[sizeof(R) == 4 ? 2 : T::NL * 4];   // FP64 form: the state
+        alignas(16) R sQf[sizeof(R) == 4 ? T::NL * 4 : 1];        // FP32 form: the compute-type state
+        alignas(16) R sJa[BR1 ? T::NL * 4 : 1];
     };
     // the state and the metric are dead once every node's gradient is formed: the gradient
     // tile takes their place
     union {
         Inputs in;
-        alignas(16) R sDQ[T::NN * ST::DS];
+        alignas(16) R sDQ[T::NL * 8];
     } u;
     alignas(16) double sLb[2 * P];
     alignas(16) R sFu[BR1 ? T::NF * 6 : 1];
@@ -426,19 +502,18 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
     const Phys<R> ph(a.ph);
     if (t < 2 * P) { sLb[t] = a.lb[t]; sLbw[t] = (R)a.lbw[t]; sLbw[2 * P + t] = (R)a.lb[t]; }
     for (int x = t; x < PP; x += TPB) {
-        if (BR1) sHat[x] = (R)a.hatD[x];
-        else sD[x] = (R)a.D[x];
+        if (BR1) sHat[x] = (R)a.hatD[(x % P) * P + x / P];
+        else sD[x] = (R)a.D[(x % P) * P + x / P];
     }
     const int ne = min(EPB, a.K - e0);
     const int64_t nb0 = (int64_t)e0 * PP;
     constexpr bool COPY = sizeof(R) == 4;
-    using ST = GradStrides<R>;
-    constexpr int QS = ST::QS, JS = ST::JS, DS = ST::DS;
-    load_tile<R, COPY, !COPY, QS>(a, nb0, ne, PP, sQ, S.u.in.sQf, t, TPB);
+    constexpr int NL = T::NL;
+    load_tile<P, NL, R, COPY, !COPY>(a, nb0, ne, sQ, S.u.in.sQf, t, TPB);
     const R *sQr;
     if constexpr (COPY) sQr = S.u.in.sQf; else sQr = (const R *)sQ;
     // ---- hoisted global loads
-    const int s = t / PP, n = t % PP, e = e0 + s;
+    const int s = t / PP, n = t % PP, e = e0 + s, x0 = s * Layout<P>::ES, xn = Layout<P>::at(s, n);
     const bool node_active = (t < NN) && (e < a.K);
     R ijac = R(1), j11 = R(0), j12 = R(0), j21 = R(0), j22 = R(0);
     int ord = 0;
@@ -447,7 +522,8 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
         load_metric<R>(a, e, g, j11, j12, j21, j22, ijac);
         if (BR1) {
             ord = a.forder[e];
-            sJa[t * JS + 0] = j11; sJa[t * JS + 1] = j12; sJa[t * JS + 2] = j21; sJa[t * JS + 3] = j22;
+            const R jv[4] = {j11, j21, j12, j22};
+            Quads<R, NL>::put(sJa, xn, jv);
         }
     }
     const int fs = t / (4 * P), ff = (t / P) % 4, fk = t % P, fe = e0 + fs;
@@ -470,22 +546,21 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
     if (node_active) {
         const int i = n % P, j = n / P;
         if (BR1) {
-            br1_node_gradient<P, R, QS, JS>(sQr + s * PP * QS, sJa + s * PP * JS, sHat, sFu + s * 4 * P * 6, sLbw, ord, i,
-                                            j, ijac, dq);
+            br1_node_gradient<P, NL, R>(sQr, sJa, x0, sHat, sFu + s * 4 * P * 6, sLbw, ord, i, j, ijac, dq);
             if (ord >> 8) mortar_y_lift<P, R>(a.mustar + (int64_t)e * 4 * P * 8, sLbw, ord, i, j, ijac, dq);
         }
-        else ip_node_gradient<P, R, QS>(sQr + s * PP * QS, sD, i, j, j11, j12, j21, j22, ijac, dq);
+        else ip_node_gradient<P, NL, R>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dq);
     }
     __syncthreads();   // every lane is done with the state and the metric
     if (node_active) {
-#pragma unroll
-        for (int c = 0; c < 8; ++c) sDQ[t * DS + c] = dq[c];
+        Quads<R, NL>::put(sDQ, xn, dq);
+        Quads<R, NL>::put(sDQ + 4 * NL, xn, dq + 4);
     }
     __syncthreads();
     if (face_active) {
         const R muf = XB ? face_mu<R>(a, ph, fe, fr) : ph.mu;
         double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + ((int64_t)(fe * 4 + ff) * P + fk) * 8 : nullptr;
-        viscous_face_trace<P, DS, R, TR>(a, ph, fr.x, qs, sDQ + fs * PP * DS, sLb, sLbw + 2 * P, ff, fk,
+        viscous_face_trace<P, NL, R, TR>(a, ph, fr.x, qs, sDQ, fs * Layout<P>::ES, sLb, sLbw + 2 * P, ff, fk,
                                          (TR *)a.dtr_out + ((int64_t)(fe * 4 + ff) * P + fk) * VT, muf, mdq);
     }
 }
@@ -500,24 +575,24 @@ __global__ __launch_bounds__((Tile<P, EPB>::TPB)) void k_gradient(StageArgs a) {
 template <int P, int EPB, bool NS, bool IP, typename R>
 struct StageSmem {
     using T = Tile<P, EPB>;
-    alignas(16) double sQ[T::NN * 4];
+    alignas(16) double sQ[T::NL * 4];
     alignas(16) double sLb[2 * P];
     alignas(16) double sRes[4][4];
     struct Fluxes {
-        alignas(16) R sCF[T::NN * 4];          // BR1: the metric Ja during the gradient phase
-        alignas(16) R sCG[T::NN * 4];          // NS, FP32: the compute-type state until the node phase
+        alignas(16) R sCF[T::NL * 4];          // BR1: the metric Ja during the gradient phase
+        alignas(16) R sCG[T::NL * 4];          // NS, FP32: the compute-type state until the node phase
     };
     // IP: the epilogue's gradient tile takes the place of the contravariant fluxes
     union {
         Fluxes f;
-        alignas(16) R sDQ[IP ? T::NN * 8 : 1];
+        alignas(16) R sDQ[IP ? T::NL * 8 : 1];
     } u;
     alignas(16) R sF[NS && !IP ? T::NF * 6 : T::NF * 4];  // BR1: uStar fluxes during the gradient phase
     // IP gradient-face terms: the face phase's contravariant fluxes, then (same arrays) the
     // U / V lift coefficients
     alignas(16) R sU[IP ? T::NF * 4 : 1];
     alignas(16) R sV[IP ? T::NF * 4 : 1];
-    alignas(16) R sHat[T::PP];
+    alignas(16) R sHat[T::PP];          // transposed, as sD: a wavefront's reads are consecutive
     alignas(16) R sD[NS ? T::PP : 1];   // IP gradient; BR1: the Laplacian dissipation's interior gradient
     alignas(16) R sLbw[2 * P];
     alignas(16) R sDlbw[2 * P];
@@ -553,20 +628,24 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         if (IP) S.sLbR[t] = (R)a.lb[t];
     }
     for (int x = t; x < PP; x += TPB) {
-        sHat[x] = (R)a.hatD[x];
-        if (IP || (BR1 && XB)) sD[x] = (R)a.D[x];
+        const int xt = (x % P) * P + x / P;
+        sHat[x] = (R)a.hatD[xt];
+        if (IP || (BR1 && XB)) sD[x] = (R)a.D[xt];
     }
     const int ne = min(EPB, a.K - e0);
     const int64_t nb0 = (int64_t)e0 * PP;
     // NS in FP32: a compute-type copy of the state for the gradient contractions, in sCG (each
     // node lane reads its own entry once more before the node phase overwrites it)
     constexpr bool COPY = NS && sizeof(R) == 4;
-    load_tile<R, COPY>(a, nb0, ne, PP, sQ, sCG, t, TPB);
+    constexpr int NL = T::NL;
+    using NodeV = Quads<R, NL>;    // node arrays
+    using FaceV = Quads<R, NF>;    // face-node arrays
+    load_tile<P, NL, R, COPY>(a, nb0, ne, sQ, sCG, t, TPB);
     const R *sQr;
     if constexpr (COPY) sQr = sCG; else sQr = (const R *)sQ;
 
     // ---- hoisted global loads: node lane
-    const int s = t / PP, n = t % PP, e = e0 + s;
+    const int s = t / PP, n = t % PP, e = e0 + s, x0 = s * Layout<P>::ES, xn = Layout<P>::at(s, n);
     const bool node_active = (t < NN) && (e < a.K);
     const int64_t g = nb0 + s * PP + n;
     R j11 = R(0), j12 = R(0), j21 = R(0), j22 = R(0), ijac = R(1);
@@ -575,7 +654,8 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         load_metric<R>(a, e, g, j11, j12, j21, j22, ijac);
         ord = a.forder[e];
         if (BR1) {
-            sCF[t * 4 + 0] = j11; sCF[t * 4 + 1] = j12; sCF[t * 4 + 2] = j21; sCF[t * 4 + 3] = j22;
+            const R jv[4] = {j11, j21, j12, j22};
+            NodeV::put(sCF, xn, jv);
         }
     }
     // ---- hoisted global loads: face lane
@@ -607,12 +687,11 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (NS && node_active) {
         const int i = n % P, j = n / P;
         if (BR1) {
-            br1_node_gradient<P, R, 4, 4, true>(sQr + s * PP * 4, sCF + s * PP * 4, sHat, sF + s * 4 * P * 6, sLbw, ord,
-                                                i, j, ijac, dq);
+            br1_node_gradient<P, NL, R, true>(sQr, sCF, x0, sHat, sF + s * 4 * P * 6, sLbw, ord, i, j, ijac, dq);
             if (ord >> 8) mortar_y_lift<P, R>(a.mustar + (int64_t)e * 4 * P * 8, sLbw, ord, i, j, ijac, dq);
         }
-        else ip_node_gradient<P, R>(sQr + s * PP * 4, sD, i, j, j11, j12, j21, j22, ijac, dq);
-        if (LAPG && a.lap) ip_node_gradient<P, R>(sQr + s * PP * 4, sD, i, j, j11, j12, j21, j22, ijac, dqi);
+        else ip_node_gradient<P, NL, R>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dq);
+        if (LAPG && a.lap) ip_node_gradient<P, NL, R>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dqi);
     }
     // the neighbour's viscous flux trace, issued before the barrier and consumed in the face phase
     R vn[NS ? VT : 1];
@@ -639,12 +718,13 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (node_active) {
         R q[4], f[4], gg[4];
         if constexpr (COPY) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) q[c] = sQr[t * 4 + c];
+            NodeV::get(sQr, xn, q);
         } else {
+            double qd[4];
+            Quads<double, NL>::get(sQ, xn, qd);
+            qd[3] = slot_energy<R>(a.ph, qd[3]);
 #pragma unroll
-            for (int c = 0; c < 3; ++c) q[c] = (R)sQ[t * 4 + c];
-            q[3] = (R)slot_energy<R>(a.ph, sQ[t * 4 + 3]);
+            for (int c = 0; c < 4; ++c) q[c] = (R)qd[c];
         }
         inviscid_flux(ph, q, f, gg);
         if (NS) {
@@ -663,11 +743,14 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
 #pragma unroll
             for (int c = 0; c < 4; ++c) { f[c] = (f[c] - mue * fv[c]) - fa[c]; gg[c] = (gg[c] - mue * gv[c]) - ga[c]; }
         }
+        R cf[4], cg4[4];
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            sCF[t * 4 + c] = f[c] * j11 + gg[c] * j21;
-            sCG[t * 4 + c] = f[c] * j12 + gg[c] * j22;
+            cf[c] = f[c] * j11 + gg[c] * j21;
+            cg4[c] = f[c] * j12 + gg[c] * j22;
         }
+        NodeV::put(sCF, xn, cf);
+        NodeV::put(sCG, xn, cg4);
     }
 
     // ---- face phase: Riemann fluxes of the element's own four faces
@@ -676,19 +759,22 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         if (kind == FK_MORTAR) {
             // p-non-conforming edge: (Fi - Fv) dS projected to this side by the mortar kernel
             const double *mf = a.mflux + ((int64_t)(fe * 4 + ff) * P + fk) * 4;
-#pragma unroll
-            for (int c = 0; c < 4; ++c) sF[t * 4 + c] = (R)mf[c];
+            const R F[4] = {(R)mf[0], (R)mf[1], (R)mf[2], (R)mf[3]};
+            FaceV::put(sF, t, F);
             if (ipgrad) {
                 // this side's IP gradient flux, projected and times dS by the mortar kernel, in
                 // contravariant components (DGWeakIntegrals.f90:268-495)
                 const double *mg = a.mgrad + ((int64_t)(fe * 4 + ff) * P + fk) * 8;
                 const R *fm = (const R *)a.fmet + ((int64_t)(fe * 4 + ff) * P + fk) * 5;
+                R fc[4], gc[4];
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
                     const R gx = (R)mg[c], gy = (R)mg[4 + c];
-                    sU[t * 4 + c] = (gx * fm[0] + gy * fm[1]) * fm[4];
-                    sV[t * 4 + c] = (gx * fm[2] + gy * fm[3]) * fm[4];
+                    fc[c] = (gx * fm[0] + gy * fm[1]) * fm[4];
+                    gc[c] = (gx * fm[2] + gy * fm[3]) * fm[4];
                 }
+                FaceV::put(sU, t, fc);
+                FaceV::put(sV, t, gc);
             }
         } else {
             R vs[NS ? VT : 1];   // own viscous flux trace
@@ -799,19 +885,21 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                 if (ipgrad) {
                     // contravariant gradient-flux components at the face (DGWeakIntegrals.f90:268-495)
                     const R *fm = (const R *)a.fmet + ((int64_t)(fe * 4 + ff) * P + fk) * 5;
+                    R fc[4], gc[4];
 #pragma unroll
                     for (int c = 0; c < 4; ++c) {
-                        sU[t * 4 + c] = (G8[c] * fm[0] + G8[4 + c] * fm[1]) * fm[4];   // fm[4] = 1/jac at the face node
-                        sV[t * 4 + c] = (G8[c] * fm[2] + G8[4 + c] * fm[3]) * fm[4];
+                        fc[c] = (G8[c] * fm[0] + G8[4 + c] * fm[1]) * fm[4];   // fm[4] = 1/jac at the face node
+                        gc[c] = (G8[c] * fm[2] + G8[4 + c] * fm[3]) * fm[4];
                     }
+                    FaceV::put(sU, t, fc);
+                    FaceV::put(sV, t, gc);
                 }
             }
             if (kind == FK_INT_R) {
 #pragma unroll
                 for (int c = 0; c < 4; ++c) F[c] = -F[c];
             }
-#pragma unroll
-            for (int c = 0; c < 4; ++c) sF[t * 4 + c] = F[c];
+            FaceV::put(sF, t, F);
         }
     }
     __syncthreads();
@@ -821,22 +909,25 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (ipgrad) {
         R u2[4], v2[4];
         if (face_active) {
-            const R *Fc = sU + (fs * 4 + ff) * P * 4, *Gc = sV + (fs * 4 + ff) * P * 4;
             const bool horiz = (ff == 0 || ff == 2);
-            const R *src = horiz ? Fc : Gc;
+            const R *src = horiz ? sU : sV;
+            const int xf = (fs * 4 + ff) * P;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                R acc = R(0);
+            for (int c = 0; c < 4; ++c) u2[c] = R(0);
 #pragma unroll
-                for (int l = 0; l < P; ++l) acc += sHat[fk * P + l] * src[l * 4 + c];
-                u2[c] = acc;
-                v2[c] = horiz ? Gc[fk * 4 + c] : Fc[fk * 4 + c];
+            for (int l = 0; l < P; ++l) {
+                const R h = sHat[l * P + fk];
+                R v[4];
+                FaceV::get(src, xf + l, v);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) u2[c] += h * v[c];
             }
+            FaceV::get(horiz ? sV : sU, xf + fk, v2);
         }
         __syncthreads();   // every face has read its fluxes: U and V take their place
         if (face_active) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) { sU[t * 4 + c] = u2[c]; sV[t * 4 + c] = v2[c]; }
+            FaceV::put(sU, t, u2);
+            FaceV::put(sV, t, v2);
         }
         __syncthreads();
     }
@@ -852,12 +943,14 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (node_active) {
         const int i = n % P, j = n / P;
         R acc[4] = {R(0), R(0), R(0), R(0)};
-        const R *cF = sCF + s * PP * 4, *cG = sCG + s * PP * 4;
 #pragma unroll 1
         for (int l = 0; l < P; ++l) {
-            const R hi = sHat[i * P + l], hj = sHat[j * P + l];
+            const R hi = sHat[l * P + i], hj = sHat[l * P + j];
+            R cF[4], cG[4];
+            NodeV::get(sCF, x0 + l + Layout<P>::RS * j, cF);
+            NodeV::get(sCG, x0 + i + Layout<P>::RS * l, cG);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) acc[c] = acc[c] + hi * cF[(l + P * j) * 4 + c] + hj * cG[(i + P * l) * 4 + c];
+            for (int c = 0; c < 4; ++c) acc[c] = acc[c] + hi * cF[c] + hj * cG[c];
         }
 #pragma unroll
         for (int o = 0; o < 4; ++o) {
@@ -866,12 +959,16 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             const int oth = (f == 0 || f == 2) ? j : i;
             const int side = (f == 0 || f == 3) ? 0 : P;
             const R lw = sLbw[side + oth];
-            const R *Ff = sF + ((s * 4 + f) * P + idx) * 4;
+            const int xf = (s * 4 + f) * P + idx;
+            R Ff[4];
+            FaceV::get(sF, xf, Ff);
 #pragma unroll
             for (int c = 0; c < 4; ++c) acc[c] = acc[c] - Ff[c] * lw;
             if (ipgrad) {
                 const R dlw = sDlbw[side + oth];
-                const R *Uf = sU + ((s * 4 + f) * P + idx) * 4, *Vf = sV + ((s * 4 + f) * P + idx) * 4;
+                R Uf[4], Vf[4];
+                FaceV::get(sU, xf, Uf);
+                FaceV::get(sV, xf, Vf);
 #pragma unroll
                 for (int c = 0; c < 4; ++c) acc[c] = acc[c] - (Uf[c] * lw + Vf[c] * dlw);
             }
@@ -895,13 +992,13 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             go[0] = make_double2(gv[0], gv[1]);
             go[1] = make_double2(gv[2], gv[3]);
             double qn[4];
+            Quads<double, NL>::get(sQ, xn, qn);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) qn[c] = fma(cg, gv[c], sQ[t * 4 + c]);
+            for (int c = 0; c < 4; ++c) qn[c] = fma(cg, gv[c], qn[c]);
             double2 *qo2 = (double2 *)(a.Q + g * 4);
             qo2[0] = make_double2(qn[0], qn[1]);
             qo2[1] = make_double2(qn[2], qn[3]);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) sQ[t * 4 + c] = qn[c];
+            Quads<double, NL>::put(sQ, xn, qn);
         }
     }
     if (a.do_resid) {
@@ -931,7 +1028,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         R qn[4];   // the next stage's own Q trace in the compute type (IP epilogue)
         if (face_active) {
             double tq[4];
-            face_trace<P, 4, 4>(sQ + fs * PP * 4, sLb, ff, fk, tq);
+            face_trace<P, NL>(sQ, fs * Layout<P>::ES, sLb, ff, fk, tq);
             tq[3] = slot_energy<TR>(a.ph, tq[3]);
             TR *o = (TR *)a.tr_out + ((int64_t)(fe * 4 + ff) * P + fk) * 4;
 #pragma unroll
@@ -947,8 +1044,12 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             const R *sQn;
             if constexpr (COPY) {
                 if (node_active) {
+                    double qd4[4];
+                    Quads<double, NL>::get(sQ, xn, qd4);
+                    R qc[4];
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) sCG[t * 4 + c] = qslot<R>(a.ph, sQ[t * 4 + c], c);
+                    for (int c = 0; c < 4; ++c) qc[c] = qslot<R>(a.ph, qd4[c], c);
+                    NodeV::put(sCG, xn, qc);
                 }
                 __syncthreads();
                 sQn = sCG;
@@ -961,18 +1062,18 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                 // FP64 kernel a wavefront per SIMD
                 R m11, m12, m21, m22, mij;
                 load_metric<R>(a, e, g, m11, m12, m21, m22, mij);
-                ip_node_gradient<P, R>(sQn + s * PP * 4, sD, n % P, n / P, m11, m12, m21, m22, mij, dq);
+                ip_node_gradient<P, NL, R>(sQn, x0, sD, n % P, n / P, m11, m12, m21, m22, mij, dq);
             }
             __syncthreads();   // the state copy and the fluxes' space are free
             R *sDQ = S.u.sDQ;
             if (node_active) {
-#pragma unroll
-                for (int c = 0; c < 8; ++c) sDQ[t * 8 + c] = dq[c];
+                NodeV::put(sDQ, xn, dq);
+                NodeV::put(sDQ + 4 * NL, xn, dq + 4);
             }
             __syncthreads();
             if (face_active) {
                 double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + ((int64_t)(fe * 4 + ff) * P + fk) * 8 : nullptr;
-                viscous_face_trace<P, 8, R, TR>(a, ph, fr.x, qn, sDQ + fs * PP * 8, sLb, S.sLbR, ff, fk,
+                viscous_face_trace<P, NL, R, TR>(a, ph, fr.x, qn, sDQ, fs * Layout<P>::ES, sLb, S.sLbR, ff, fk,
                                                 (TR *)a.dtr_out + ((int64_t)(fe * 4 + ff) * P + fk) * VT, ph.mu, mdq);
             }
           }

@@ -1,5 +1,4 @@
-// Point-wise physics on the device: fluxes, Riemann solvers, boundary ghost states and the
-// face-trace helper shared by every kernel.  Templated on the compute type R (double for the
+// Point-wise physics on the device: fluxes, Riemann solvers and boundary ghost states.  Templated on the compute type R (double for the
 // FP64 form, float for the mixed form).
 #pragma once
 #include <hip/hip_runtime.h>
@@ -595,47 +594,6 @@ __device__ inline int ghost_state(int kind, int flags, const double *zd, const P
                      : Qt[3] - Ek + R(0.5) * uSB[0] * (vwx * vwx + vwy * vwy);
     }
     return 0;
-}
-
-// ------------------------------------------------------------------ spectral helpers
-// Trace of a face from the staged element state (DGSpatialDiscretizationMethods.f90:1520-1574).
-// Always accumulated in FP64 with explicit fma in l order so that every kernel that forms
-// a trace (prolong, stage epilogue, stage recomputation) produces the same bits.
-template <int P, int STRIDE, int NV, typename T>
-__device__ inline void face_trace(const T *sX /* element block, [n*STRIDE + c] */, const double *sLb, int f, int k,
-                                  double *out) {
-    const double *lb = (f == 0 || f == 3) ? sLb : sLb + P;
-    // nodes (k, l) of a horizontal face or (l, k) of a vertical one: a base and a stride, so
-    // the loop body has no face-dependent branch
-    const bool horiz = (f == 0 || f == 2);
-    const int base = horiz ? k : P * k, step = horiz ? P : 1;
-#pragma unroll
-    for (int c = 0; c < NV; ++c) out[c] = 0.0;
-    // a rolled loop keeps one node's values live (unrolled, all P nodes are loaded up front)
-#pragma unroll 1
-    for (int l = 0; l < P; ++l) {
-        const int n = base + step * l;
-#pragma unroll
-        for (int c = 0; c < NV; ++c) out[c] = fma((double)sX[n * STRIDE + c], lb[l], out[c]);
-    }
-}
-
-// face_trace accumulated in the tile's own type.  The FP32 form uses it for the gradient
-// traces, which only the kernel that forms them ever evaluates (the viscous face fluxes are
-// stored), so no other kernel needs to reproduce these bits.
-template <int P, int STRIDE, int NV, typename T>
-__device__ inline void face_trace_r(const T *sX, const T *sLb, int f, int k, T *out) {
-    const T *lb = (f == 0 || f == 3) ? sLb : sLb + P;
-    const bool horiz = (f == 0 || f == 2);
-    const int base = horiz ? k : P * k, step = horiz ? P : 1;
-#pragma unroll
-    for (int c = 0; c < NV; ++c) out[c] = T(0);
-#pragma unroll 1
-    for (int l = 0; l < P; ++l) {
-        const int n = base + step * l;
-#pragma unroll
-        for (int c = 0; c < NV; ++c) out[c] = fma(sX[n * STRIDE + c], lb[l], out[c]);
-    }
 }
 
 }  // namespace hg
