@@ -165,21 +165,27 @@ struct Tiles {
     static constexpr int large = (wide < lds_cap ? wide : lds_cap) > 0 ? (wide < lds_cap ? wide : lds_cap) : 1;
 };
 
-// Stages an element tile's state from HBM into LDS: FP64 (KEEP64), plus the compute-type copy
-// (energy slot shifted) that the gradient contractions read when the compute type is FP32.
-template <int P, int NL, typename R, bool COPY, bool KEEP64 = true>
-__device__ __forceinline__ void load_tile(const StageArgs &a, const int64_t nb0, const int ne, double *sQ, R *sQf,
-                                          const int t, const int TPB) {
-    constexpr int PP = P * P;
-    const double2 *src = (const double2 *)(a.Q + nb0 * 4);
-    for (int x = t; x < ne * PP * 2; x += TPB) {
-        // pairs (0, 1) and (2, 3) of a node: the odd pair holds the energy
-        const double2 v = src[x];
-        const int h = x & 1, e = Layout<P>::at((x >> 1) / PP, (x >> 1) % PP);
-        if constexpr (KEEP64) *(double2 *)(sQ + 2 * NL * h + 2 * e) = v;
-        if constexpr (COPY)
-            *(float2 *)(sQf + 4 * e + 2 * h) = make_float2((float)v.x, (float)(h ? slot_energy<R>(a.ph, v.y) : v.y));
-    }
+// The state of node g: each lane reads its own node's 32 bytes, so no lane waits for another's
+// before it has its own.
+__device__ __forceinline__ void load_node(const double *Q, int64_t g, double *q) {
+    const double2 *p = (const double2 *)(Q + g * 4);
+    const double2 a = p[0], b = p[1];
+    q[0] = a.x; q[1] = a.y; q[2] = b.x; q[3] = b.y;
+}
+
+// The state slot the compute type sees (energy shifted in the FP32 form).
+template <typename R>
+__device__ __forceinline__ R qslot(const PhysParams &pp, double v, int c) {
+    return (R)(c == 3 ? slot_energy<R>(pp, v) : v);
+}
+
+// The compute-type copy of a node's state that the FP32 form's gradient contractions read.
+template <int NL, typename R>
+__device__ __forceinline__ void put_slots(const PhysParams &pp, R *sQf, int x, const double *q) {
+    R v[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = qslot<R>(pp, q[c], c);
+    Quads<R, NL>::put(sQf, x, v);
 }
 
 // ------------------------------------------------------------------ prolongation
@@ -190,7 +196,11 @@ __global__ __launch_bounds__((Tile<P, EPB>::TPB)) void k_prolong(StageArgs a) {
     __shared__ double sLb[2 * P];
     const int t = threadIdx.x, e0 = blockIdx.x * EPB;
     if (t < 2 * P) sLb[t] = a.lb[t];
-    load_tile<P, T::NL, double, false>(a, (int64_t)e0 * T::PP, min(EPB, a.K - e0), sQ, (double *)nullptr, t, T::TPB);
+    if (t < T::NN && e0 + t / T::PP < a.K) {
+        double q[4];
+        load_node(a.Q, (int64_t)e0 * T::PP + t, q);
+        Quads<double, T::NL>::put(sQ, Layout<P>::at(t / T::PP, t % T::PP), q);
+    }
     __syncthreads();
     if (t < T::NF) {
         const int s = t / (4 * P), f = (t / P) % 4, k = t % P, e = e0 + s;
@@ -209,12 +219,6 @@ __global__ __launch_bounds__((Tile<P, EPB>::TPB)) void k_prolong(StageArgs a) {
 // Both the trace kernel (k_gradient) and the stage kernel evaluate the element gradient with
 // these functions, so the gradient a stage recomputes for its own element is the one whose
 // face traces its neighbours read.
-
-// The state slot the compute type sees (energy shifted in the FP32 form).
-template <typename R>
-__device__ __forceinline__ R qslot(const PhysParams &pp, double v, int c) {
-    return (R)(c == 3 ? slot_energy<R>(pp, v) : v);
-}
 
 // The state a boundary face node's ghost state starts from: its zone's record (8 doubles per
 // zone, the state in the first four), or, on a face flagged FF_FSTATE, the node's own value of
@@ -505,11 +509,9 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
         if (BR1) sHat[x] = (R)a.hatD[(x % P) * P + x / P];
         else sD[x] = (R)a.D[(x % P) * P + x / P];
     }
-    const int ne = min(EPB, a.K - e0);
     const int64_t nb0 = (int64_t)e0 * PP;
     constexpr bool COPY = sizeof(R) == 4;
     constexpr int NL = T::NL;
-    load_tile<P, NL, R, COPY, !COPY>(a, nb0, ne, sQ, S.u.in.sQf, t, TPB);
     const R *sQr;
     if constexpr (COPY) sQr = S.u.in.sQf; else sQr = (const R *)sQ;
     // ---- hoisted global loads
@@ -519,7 +521,11 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
     int ord = 0;
     if (node_active) {
         const int64_t g = nb0 + s * PP + n;
+        double qg[4];
+        load_node(a.Q, g, qg);
         load_metric<R>(a, e, g, j11, j12, j21, j22, ijac);
+        if constexpr (COPY) put_slots<NL, R>(a.ph, S.u.in.sQf, xn, qg);
+        else Quads<double, NL>::put(sQ, xn, qg);
         if (BR1) {
             ord = a.forder[e];
             const R jv[4] = {j11, j21, j12, j22};
@@ -537,11 +543,10 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
         else fr = a.face[fe * 4 + ff];
         stored_trace<P, R, TR>(a, fe, ff, fk, qs);
     }
-    __syncthreads();
     if (BR1 && face_active)
         br1_face_flux<R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx, ny,
                              dS, sFu + t * 6);
-    if (BR1) __syncthreads();
+    __syncthreads();
     R dq[8];
     if (node_active) {
         const int i = n % P, j = n / P;
@@ -632,7 +637,6 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         sHat[x] = (R)a.hatD[xt];
         if (IP || (BR1 && XB)) sD[x] = (R)a.D[xt];
     }
-    const int ne = min(EPB, a.K - e0);
     const int64_t nb0 = (int64_t)e0 * PP;
     // NS in FP32: a compute-type copy of the state for the gradient contractions, in sCG (each
     // node lane reads its own entry once more before the node phase overwrites it)
@@ -640,7 +644,6 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     constexpr int NL = T::NL;
     using NodeV = Quads<R, NL>;    // node arrays
     using FaceV = Quads<R, NF>;    // face-node arrays
-    load_tile<P, NL, R, COPY>(a, nb0, ne, sQ, sCG, t, TPB);
     const R *sQr;
     if constexpr (COPY) sQr = sCG; else sQr = (const R *)sQ;
 
@@ -650,9 +653,16 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     const int64_t g = nb0 + s * PP + n;
     R j11 = R(0), j12 = R(0), j21 = R(0), j22 = R(0), ijac = R(1);
     int ord = 0;
+    // the own node's state: staged in LDS for the gradient contractions (Navier-Stokes) and for
+    // the update; the Euler form takes its flux from the registers, so nothing there waits for
+    // another lane until the fluxes are formed
+    double qg[4];
     if (node_active) {
+        load_node(a.Q, g, qg);
         load_metric<R>(a, e, g, j11, j12, j21, j22, ijac);
         ord = a.forder[e];
+        Quads<double, NL>::put(sQ, xn, qg);
+        if constexpr (COPY) put_slots<NL, R>(a.ph, sCG, xn, qg);
         if (BR1) {
             const R jv[4] = {j11, j21, j12, j22};
             NodeV::put(sCF, xn, jv);
@@ -669,14 +679,10 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         load_face<P, R, TR>(a, fe, ff, fk, fr, nx, ny, dS, qo, nslot);
         stored_trace<P, R, TR>(a, fe, ff, fk, qs);
     }
-    __syncthreads();
-
-    if (BR1) {
-        if (face_active)
-            br1_face_flux<R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx,
-                                 ny, dS, sF + t * 6);
-        __syncthreads();
-    }
+    if (BR1 && face_active)
+        br1_face_flux<R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx, ny,
+                             dS, sF + t * 6);
+    if (NS) __syncthreads();
 
     // ---- own nodal gradient (Navier-Stokes), kept in registers for the node phase
     R dq[NS ? 8 : 1];
@@ -720,11 +726,9 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         if constexpr (COPY) {
             NodeV::get(sQr, xn, q);
         } else {
-            double qd[4];
-            Quads<double, NL>::get(sQ, xn, qd);
-            qd[3] = slot_energy<R>(a.ph, qd[3]);
+            if (NS) Quads<double, NL>::get(sQ, xn, qg);
 #pragma unroll
-            for (int c = 0; c < 4; ++c) q[c] = (R)qd[c];
+            for (int c = 0; c < 4; ++c) q[c] = qslot<R>(a.ph, qg[c], c);
         }
         inviscid_flux(ph, q, f, gg);
         if (NS) {
@@ -1044,12 +1048,9 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             const R *sQn;
             if constexpr (COPY) {
                 if (node_active) {
-                    double qd4[4];
-                    Quads<double, NL>::get(sQ, xn, qd4);
-                    R qc[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) qc[c] = qslot<R>(a.ph, qd4[c], c);
-                    NodeV::put(sCG, xn, qc);
+                    double qu[4];
+                    Quads<double, NL>::get(sQ, xn, qu);
+                    put_slots<NL, R>(a.ph, sCG, xn, qu);
                 }
                 __syncthreads();
                 sQn = sCG;
