@@ -34,7 +34,37 @@ namespace hg {
 template <typename T>
 __device__ inline T ld(const void *p, int64_t i) { return ((const T *)p)[i]; }
 
-__device__ inline double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }
+// Per equation, the maximum of |q| over a wavefront's lanes, every lane active.  Lane l returns that of value wave_max4_value(l).  Magnitudes compare as the unsigned
+// integers of their bits, where a NaN is above infinity.  Two steps within the quads halve the values
+// a lane carries, so each of the other four exchanges one value instead of four: 10 cross-lane moves
+// of 32 bits against the 48 of a shuffle tree per value, which made the last stage of a step 10 %
+// longer than the others (148 against 135 us on an ensemble of 16 M unknowns, 235 against 214 us on
+// the 256 x 256 interior-penalty mesh).
+__device__ __forceinline__ int wave_max4_value(int l) { return 2 * (l & 1) + ((l >> 1) & 1); }
+
+template <int CTRL>
+__device__ __forceinline__ uint64_t dpp_move(uint64_t v) {
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, CTRL, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), CTRL, 0xf, 0xf, false);
+    return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
+}
+
+__device__ __forceinline__ uint64_t wave_max4(const double *q) {
+    uint64_t v[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = (uint64_t)__double_as_longlong(fabs(q[c]));
+    const int l = threadIdx.x;
+    constexpr int QUAD_XOR1 = 0xB1, QUAD_XOR2 = 0x4E, ROW_ROR4 = 0x124, ROW_ROR8 = 0x128;
+    const bool odd = l & 1, up = l & 2;
+    // even lanes keep values 0, 1 and hand over 2, 3
+    const uint64_t r0 = dpp_move<QUAD_XOR1>(odd ? v[0] : v[2]), r1 = dpp_move<QUAD_XOR1>(odd ? v[1] : v[3]);
+    const uint64_t p0 = max(odd ? v[2] : v[0], r0), p1 = max(odd ? v[3] : v[1], r1);
+    uint64_t m = max(up ? p1 : p0, dpp_move<QUAD_XOR2>(up ? p0 : p1));
+    m = max(m, dpp_move<ROW_ROR4>(m));
+    m = max(m, dpp_move<ROW_ROR8>(m));
+    m = max(m, (uint64_t)__shfl_xor((unsigned long long)m, 16, 64));
+    return max(m, (uint64_t)__shfl_xor((unsigned long long)m, 32, 64));
+}
 
 // Tile handled by workgroup b of nb.  The dispatcher hands consecutive workgroups to the eight
 // XCDs in turn; this gives each XCD a contiguous range of tiles (a band of the mesh), so that
@@ -582,7 +612,7 @@ struct StageSmem {
     using T = Tile<P, EPB>;
     alignas(16) double sQ[T::NL * 4];
     alignas(16) double sLb[2 * P];
-    alignas(16) double sRes[4][4];
+    alignas(16) uint64_t sRes[4][4];
     struct Fluxes {
         alignas(16) R sCF[T::NL * 4];          // BR1: the metric Ja during the gradient phase
         alignas(16) R sCG[T::NL * 4];          // NS, FP32: the compute-type state until the node phase
@@ -992,9 +1022,12 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
 #pragma unroll
                 for (int c = 0; c < 4; ++c) gv[c] = fma(a.am, gold[c], cq * qd[c]);
             }
-            double2 *go = (double2 *)(a.G + g * 4);
-            go[0] = make_double2(gv[0], gv[1]);
-            go[1] = make_double2(gv[2], gv[3]);
+            // the last stage's register is read by nobody: the next step's first stage starts it anew
+            if (!a.do_resid) {
+                double2 *go = (double2 *)(a.G + g * 4);
+                go[0] = make_double2(gv[0], gv[1]);
+                go[1] = make_double2(gv[2], gv[3]);
+            }
             double qn[4];
             Quads<double, NL>::get(sQ, xn, qn);
 #pragma unroll
@@ -1005,30 +1038,19 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             Quads<double, NL>::put(sQ, xn, qn);
         }
     }
+    // max|QDot| per equation: across the wavefront here, across the workgroup's wavefronts after the
+    // barrier; one partial per workgroup (reduced by k_resid_final)
     if (a.do_resid) {
-        // max|QDot| per equation: wavefront shuffle, then across the workgroup's wavefronts in
-        // LDS; one partial per workgroup (reduced by k_resid_final).  NaN wins every compare.
-        double(*sRes)[4] = S.sRes;
-        double m[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            double v = node_active ? fabs(qd[c]) : 0.0;
-            for (int off = 32; off > 0; off >>= 1) v = nan_max(v, __shfl_xor(v, off, 64));
-            m[c] = v;
-        }
-        if ((t & 63) == 0) {
-#pragma unroll
-            for (int c = 0; c < 4; ++c) sRes[t >> 6][c] = m[c];
-        }
-        __syncthreads();
-        if (t < 4) {
-            double v = sRes[0][t];
-            for (int w = 1; w < TPB / 64; ++w) v = nan_max(v, sRes[w][t]);
-            a.resid_part[rslot * 4 + t] = v;
-        }
+        const uint64_t m = wave_max4(qd);   // zeros where the lane has no node
+        if ((t & 63) < 4) S.sRes[t >> 6][t & 3] = m;
+    }
+    if (a.do_resid || a.mode == 0) __syncthreads();
+    if (a.do_resid && t < 4) {
+        uint64_t v = S.sRes[0][t];
+        for (int w = 1; w < TPB / 64; ++w) v = max(v, S.sRes[w][t]);
+        a.resid_part[rslot * 4 + wave_max4_value(t)] = __longlong_as_double((long long)v);
     }
     if (a.mode == 0) {
-        __syncthreads();
         R qn[4];   // the next stage's own Q trace in the compute type (IP epilogue)
         if (face_active) {
             double tq[4];
