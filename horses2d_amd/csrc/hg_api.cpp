@@ -58,6 +58,34 @@ hipError_t upload_real(hg_handle *h, void **dst, const std::vector<double> &src,
     return e;
 }
 
+// The metric planes (Ja11, Ja12, Ja21, Ja22, 1/jac per node) as two values per line of nodes,
+// (Ja11, Ja21) by i and then (Ja12, Ja22) by j, if that loses no bit: straight-sided elements,
+// whose bilinear map's derivatives along one coordinate depend on the other alone.  The kernels
+// form 1/jac from them in the operations checked here.
+bool line_metric(const std::vector<double> &metric, int K, int P, std::vector<double> &lines) {
+    const size_t nn = metric.size() / 5, half = 2 * (size_t)K * P;
+    const double *M[5];
+    for (int c = 0; c < 5; ++c) M[c] = metric.data() + c * nn;
+    lines.resize(2 * half);
+    for (int e = 0; e < K; ++e) {
+        const size_t g0 = (size_t)e * P * P, l0 = 2 * (size_t)e * P;
+        for (int k = 0; k < P; ++k) {
+            lines[l0 + 2 * k] = M[0][g0 + k];
+            lines[l0 + 2 * k + 1] = M[2][g0 + k];
+            lines[half + l0 + 2 * k] = M[1][g0 + (size_t)P * k];
+            lines[half + l0 + 2 * k + 1] = M[3][g0 + (size_t)P * k];
+        }
+        for (int n = 0; n < P * P; ++n) {
+            const double *li = &lines[l0 + 2 * (n % P)], *lj = &lines[half + l0 + 2 * (n / P)];
+            const double a = lj[1] * li[0], b = li[1] * lj[0];
+            const double rec[5] = {li[0], lj[0], li[1], lj[1], 1.0 / (a - b)};
+            for (int c = 0; c < 5; ++c)
+                if (std::memcmp(&rec[c], &M[c][g0 + n], sizeof(double)) != 0) return false;
+        }
+    }
+    return true;
+}
+
 hg::StageArgs base_args(hg_handle *h) {
     hg::StageArgs a{};
     a.K = h->K;
@@ -68,7 +96,7 @@ hg::StageArgs base_args(hg_handle *h) {
     a.dtr = h->dtr[h->ip_fused ? h->cur : 0];
     a.dtr_out = h->dtr[h->ip_fused ? h->cur : 0];
     a.metric = h->metric;
-    a.metric_elem = h->metric_elem;
+    a.metric_kind = h->metric_kind;
     a.face = h->face;
     a.forder = h->forder;
     a.egeo = h->egeo;
@@ -662,10 +690,12 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
             metric_e.resize(5 * (size_t)K);
             for (int c = 0; c < 5; ++c)
                 for (int e = 0; e < K; ++e) metric_e[(size_t)c * K + e] = metric[c * nn + (size_t)e * PP];
-            h->metric_elem = 1;
+            h->metric_kind = hg::METRIC_ELEM;
         }
+    } else if (line_metric(metric, K, P, metric_e)) {
+        h->metric_kind = hg::METRIC_LINE;
     }
-    HG_CHECK(upload_real(h, &h->metric, h->metric_elem ? metric_e : metric, h->mixed));
+    HG_CHECK(upload_real(h, &h->metric, h->metric_kind == hg::METRIC_NODE ? metric : metric_e, h->mixed));
     if (!fmet.empty()) HG_CHECK(upload_real(h, &h->fmet, fmet, h->mixed));
     HG_CHECK(upload(h, &h->face, face));
     HG_CHECK(upload(h, &h->forder, forder));

@@ -37,6 +37,10 @@ constexpr int FF_MCURVED = 1 << 14;  // mortar face of a curved edge: BR1 uStar 
 // own Q and gradient traces, (f1, f2, f3, g2, g3) and one pad (f0 = g0 = 0, g1 = f2).
 constexpr int VT = 6;
 
+// How a handle's metric is stored (load_metric): per node, per element (FP32 form, every element's
+// metric constant), per line of nodes (FP64 form, every element straight-sided).
+enum MetricKind : int { METRIC_NODE = 0, METRIC_ELEM = 1, METRIC_LINE = 2 };
+
 struct PhysParams {
     double gamma, gm1, cp, cv, lambda, invSGM, mu, cpPr, sigma0, ip_eps, mach_sqrtg;
     // Reference pressure of the FP32 form (pref, Eref = pref/(gamma-1)); zero in the FP64 form.
@@ -61,8 +65,9 @@ struct StageArgs {
     void *tr_out;               // next-stage Q traces
     const void *dtr;            // viscous face-flux traces [(e*4+f)*P + k][VT] (FP64 or FP32)
     void *dtr_out;
-    const void *metric;         // 5 planes: Ja11, Ja12, Ja21, Ja22, 1/jac, per node or per element
-    int metric_elem;            // 1: one metric record per element (element-constant metric)
+    const void *metric;         // 5 planes: Ja11, Ja12, Ja21, Ja22, 1/jac, per node or per element,
+    int metric_kind;            // METRIC_NODE or METRIC_ELEM; METRIC_LINE: (Ja11, Ja21) at [e*P + i],
+                                // then (Ja12, Ja22) at [e*P + j]
     const int4 *face;           // per element face record
     const int *forder;          // per element: faces sorted by global edge id (2 bits each)
     const double *egeo;         // edge geometry triplets (nx, ny, dS)

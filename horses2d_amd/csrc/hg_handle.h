@@ -42,7 +42,7 @@ struct hg_handle {
     bool ip_fused = false;
     bool vtr_valid = false;
     void *metric = nullptr, *fmet = nullptr;
-    int metric_elem = 0;   // metric stored per element (FP32 form, element-constant metric)
+    int metric_kind = hg::METRIC_NODE;
     int4 *face = nullptr;
     int *forder = nullptr;
     double *egeo = nullptr, *einvh = nullptr, *zone = nullptr;
