@@ -274,13 +274,15 @@ int run_stage(hg_handle *h, double am, double cq, double cg, bool first, bool la
     a.first_stage = first ? 1 : 0;
     a.mode = mode;
     a.do_resid = last ? 1 : 0;
+    const int blocks = hg::stage_blocks(h->P, h->tile[0], h->K);
+    const bool atomic = mode == 0 && !(first && last) && blocks <= hg::kResidAtomic;
+    if (atomic && (first || last)) a.resid_max = h->resid;
     a.dt_dev = dt_dev;
     a.dt_cq = dt_cq;
     a.dt_cg = dt_cg;
     HG_CHECK(timed(h, 0, [&] { return hg::launch_stage(h->P, h->tile[0], h->mixed, a, h->stream); }));
-    if (last)
-        HG_CHECK(hg::launch_resid_final(h->resid_part, hg::stage_blocks(h->P, h->tile[0], h->K), h->resid, h->stream,
-                                        h->resid_scratch));
+    if (last && !atomic)
+        HG_CHECK(hg::launch_resid_final(h->resid_part, blocks, h->resid, h->stream, h->resid_scratch));
     if (mode == 0) h->cur ^= 1;
     return 0;
 }
@@ -757,10 +759,10 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
         HG_CHECK(h->alloc(&h->monitor_out, 12));
     }
     HG_CHECK(h->alloc(&h->dt_dev, 1));
-    HG_CHECK(h->alloc(&h->resid, 4));
+    HG_CHECK(h->alloc(&h->resid, 4 * hg::kResidStride));
     HG_CHECK(h->alloc(&h->resid_part, 4 * (size_t)K));   // at least one element per workgroup
     HG_CHECK(h->alloc(&h->resid_scratch, 4 * (size_t)hg::kResidGroups));
-    HG_CHECK(hipMemset(h->resid, 0, 4 * sizeof(double)));
+    HG_CHECK(hipMemset(h->resid, 0, 4 * hg::kResidStride * sizeof(double)));
     HG_CHECK(hipMemset(h->Q, 0, h->ndof * sizeof(double)));
     HG_CHECK(hipMemset(h->G, 0, h->ndof * sizeof(double)));
     HG_CHECK(hipMemset(h->QDot, 0, h->ndof * sizeof(double)));
@@ -1246,8 +1248,10 @@ int hg_residuals(hg_handle *h, double res[4]) {
         }
         return 0;
     }
-    HG_CHECK(hipMemcpyAsync(res, h->resid, 4 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
+    double r[3 * hg::kResidStride + 1];
+    HG_CHECK(hipMemcpyAsync(r, h->resid, sizeof(r), hipMemcpyDeviceToHost, h->stream));
     HG_CHECK(hipStreamSynchronize(h->stream));
+    for (int c = 0; c < 4; ++c) res[c] = r[c * hg::kResidStride];
     return 0;
 }
 

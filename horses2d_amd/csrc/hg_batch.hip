@@ -89,6 +89,7 @@ struct hg_batch {
     int2 *ranges[2] = {nullptr, nullptr};  // per tile: per case residual partial range
     double **resid_out = nullptr;          // per case: the handle's residual slots
     double *dt = nullptr;                  // per case
+    std::vector<double> dt_host;           // what dt holds (empty: not known)
     double *resid_part = nullptr;
     int tile = -1, order = -1;
     int parity = 0;
@@ -575,7 +576,12 @@ int hg_batch_rk_step(hg_batch *b, const double *t, const double *dt) {
         if (b->cases[0]->ph.ad) drop_graphs(b);
         b->parity = 0;
     }
-    HB_CHECK(hipMemcpyAsync(b->dt, dt, b->cases.size() * sizeof(double), hipMemcpyHostToDevice, b->stream));
+    // the steps read dt from the device: copied when it changes (4.6 us of a 130 us step otherwise)
+    if (b->dt_host.size() != b->cases.size() || !std::equal(b->dt_host.begin(), b->dt_host.end(), dt)) {
+        b->dt_host.clear();
+        HB_CHECK(hipMemcpyAsync(b->dt, dt, b->cases.size() * sizeof(double), hipMemcpyHostToDevice, b->stream));
+        b->dt_host.assign(dt, dt + b->cases.size());
+    }
     if (b->tile < 0) {
         if (b->parity != 0) return hg::handle_error("hg_batch_rk_step: internal parity error");
         if (autotune(b)) return 1;

@@ -54,6 +54,13 @@ struct PhysParams {
     double ad_ceps; // its intensity
 };
 
+// A handle's four residual maxima lie this many doubles apart.
+constexpr int kResidStride = 32;
+// Steps whose last stage has at most this many workgroups raise the maxima with atomics; beyond,
+// a launch of its own reduces per-workgroup partials.  A same-address atomic takes about 10 ns, a
+// launch 4 us.
+constexpr int kResidAtomic = 256;
+
 // Everything a stage or gradient kernel reads or writes.  Uniform P per handle.
 struct StageArgs {
     int K;                      // elements
@@ -82,6 +89,8 @@ struct StageArgs {
     int mode;                   // 0: RK update + next traces, 1: derivative only
     double *resid_part;         // per workgroup max|QDot| per equation (4 doubles per workgroup)
     int do_resid;
+    double *resid_max;          // or null: the maxima themselves (kResidStride apart), cleared by a
+                                // stage without do_resid and raised atomically by the one with it
     PhysParams ph;
     const double *mu_a;         // artificial viscosity per element (null: none)
     const double *lap;          // Laplacian dissipation: the indicator's viscosity per element (null: none)
@@ -212,8 +221,9 @@ hipError_t launch_stage(int P, int tile, bool mixed, const StageArgs &a, hipStre
 hipError_t launch_gradient(int P, int tile, bool mixed, const StageArgs &a, hipStream_t s);
 // Workgroups of the stage kernel (= residual partials it writes) for a tile choice.
 int stage_blocks(int P, int tile, int K);
-// Reduces nb residual partials to out[4] (NaN propagates); with scratch (4 * kResidGroups
+// Reduces nb residual partials to four maxima (NaN propagates); with scratch (4 * kResidGroups
 // doubles) many partials are reduced by several workgroups first.
+// The maxima lie kResidStride doubles apart (channels of their own for the atomics of resid_max).
 constexpr int kResidGroups = 256;
 hipError_t launch_resid_final(const double *part, int nb, double *out, hipStream_t s, double *scratch = nullptr);
 

@@ -15,18 +15,18 @@ namespace {
 
 __device__ inline double nan_max(double a, double b) { return (b > a || b != b) ? b : a; }
 
-// max|QDot| per equation over the stage kernel's per-workgroup partials (4 doubles each):
-// workgroup g takes the partials g*1024 + t, stepping by the grid, every lane keeping four
-// partials' loads in flight, then wavefront shuffles and LDS; it writes its four maxima to
-// out[4 g].  The maximum does not depend on the order (NaN wins every compare), so the result
-// is exact whatever the grid.
-__global__ __launch_bounds__(1024) void k_resid_final(const double *part, int nb, double *out) {
+// max|QDot| per equation over n residual partials (4 doubles each), by one workgroup of 1024
+// lanes: partials first + t, stepping by stride, every lane keeping four partials' loads in
+// flight, then wavefront shuffles and LDS; the four maxima go to out[stride_out c].  The maximum does
+// not depend on the order (NaN wins every compare), so the result is exact whatever the grid.
+__device__ __forceinline__ void max_partials(const double *part, int n, int first, int stride, double *out,
+                                             int stride_out) {
     __shared__ double s[16][4];
-    const int t = threadIdx.x, stride = 1024 * gridDim.x;
+    const int t = threadIdx.x;
     const double2 *p2 = (const double2 *)part;
     double m[4] = {0.0, 0.0, 0.0, 0.0};
-    int b = blockIdx.x * 1024 + t;
-    for (; b + 3 * stride < nb; b += 4 * stride) {
+    int b = first + t;
+    for (; b + 3 * stride < n; b += 4 * stride) {
         double2 v[8];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
@@ -39,7 +39,7 @@ __global__ __launch_bounds__(1024) void k_resid_final(const double *part, int nb
             m[2] = nan_max(m[2], v[2 * u + 1].x); m[3] = nan_max(m[3], v[2 * u + 1].y);
         }
     }
-    for (; b < nb; b += stride) {
+    for (; b < n; b += stride) {
         const double2 a = p2[(int64_t)b * 2], c = p2[(int64_t)b * 2 + 1];
         m[0] = nan_max(m[0], a.x); m[1] = nan_max(m[1], a.y); m[2] = nan_max(m[2], c.x); m[3] = nan_max(m[3], c.y);
     }
@@ -54,8 +54,13 @@ __global__ __launch_bounds__(1024) void k_resid_final(const double *part, int nb
     if (t < 4) {
         double v = s[0][t];
         for (int w = 1; w < 16; ++w) v = nan_max(v, s[w][t]);
-        out[blockIdx.x * 4 + t] = v;
+        out[t * stride_out] = v;
     }
+}
+
+// Workgroup g of the grid reduces its share of the partials to out + 4 g.
+__global__ __launch_bounds__(1024) void k_resid_final(const double *part, int nb, double *out, int stride_out) {
+    max_partials(part, nb, blockIdx.x * 1024, 1024 * gridDim.x, out + blockIdx.x * 4, stride_out);
 }
 
 // TimeIntegrator_EstimateTimeStep (DGTimeIntegrator.f90:462-511), second half: the running
@@ -191,22 +196,10 @@ __global__ __launch_bounds__(64) void k_probes(const double *Q, const double *QD
     out[k] = o;
 }
 
-// Residual of each case of a batch: max over its tiles' partials (NaN propagates).
-__global__ __launch_bounds__(256) void k_batch_resid(const double *part, const int2 *ranges, double *const *out) {
-    __shared__ double s[256][4];
-    const int t = threadIdx.x, c = blockIdx.x;
-    const int2 r = ranges[c];
-    double m[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int b = r.x + t; b < r.y; b += 256)
-        for (int q = 0; q < 4; ++q) m[q] = nan_max(m[q], part[(int64_t)b * 4 + q]);
-    for (int q = 0; q < 4; ++q) s[t][q] = m[q];
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w)
-            for (int q = 0; q < 4; ++q) s[t][q] = nan_max(s[t][q], s[t + w][q]);
-        __syncthreads();
-    }
-    if (t < 4) out[c][t] = s[0][t];
+// Residual of each case of a batch (one workgroup): the maxima of its tiles' partials.
+__global__ __launch_bounds__(1024) void k_batch_resid(const double *part, const int2 *ranges, double *const *out) {
+    const int2 r = ranges[blockIdx.x];
+    max_partials(part + (int64_t)r.x * 4, r.y - r.x, 0, 1024, out[blockIdx.x], kResidStride);
 }
 
 }  // namespace
@@ -263,18 +256,18 @@ hipError_t launch_gradient(int P, int tile, bool mixed, const StageArgs &a, hipS
 }
 
 hipError_t launch_resid_final(const double *part, int nb, double *out, hipStream_t st, double *scratch) {
-    // one workgroup (one lane per partial) when that covers them; beyond, a first pass of up to
-    // kResidGroups workgroups into scratch, then one workgroup over their maxima (one workgroup
-    // over 64 k partials, the 256 x 256 order-7 mesh, took 37 us of a 250 us stage)
+    // one workgroup up to 8 partials per lane; beyond, a first pass of up to kResidGroups
+    // workgroups into scratch, then one workgroup over their maxima (one workgroup over 64 k
+    // partials took 37 us, two launches take 9, one over 3.3 k partials 4.5)
     const int groups = std::min(kResidGroups, (nb + 1023) / 1024);
-    if (groups <= 1 || !scratch) {
-        hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(1024), 0, st, part, nb, out);
+    if (groups <= 8 || !scratch) {
+        hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(1024), 0, st, part, nb, out, kResidStride);
         return hipGetLastError();
     }
-    hipLaunchKernelGGL(k_resid_final, dim3(groups), dim3(1024), 0, st, part, nb, scratch);
+    hipLaunchKernelGGL(k_resid_final, dim3(groups), dim3(1024), 0, st, part, nb, scratch, 1);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(1024), 0, st, scratch, groups, out);
+    hipLaunchKernelGGL(k_resid_final, dim3(1), dim3(1024), 0, st, scratch, groups, out, kResidStride);
     return hipGetLastError();
 }
 
@@ -483,7 +476,7 @@ hipError_t launch_batch_gradient_p(int variant, int P, int tile, const BatchArgs
 }
 
 hipError_t launch_batch_resid(const double *part, const int2 *ranges, double *const *out, int ncases, hipStream_t st) {
-    hipLaunchKernelGGL(k_batch_resid, dim3(ncases), dim3(256), 0, st, part, ranges, out);
+    hipLaunchKernelGGL(k_batch_resid, dim3(ncases), dim3(1024), 0, st, part, ranges, out);
     return hipGetLastError();
 }
 

@@ -1059,7 +1059,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         }
     }
     // max|QDot| per equation: across the wavefront here, across the workgroup's wavefronts after the
-    // barrier; one partial per workgroup (reduced by k_resid_final)
+    // barrier; one partial per workgroup (reduced by k_resid_final), or one atomic maximum
     if (a.do_resid) {
         const uint64_t m = wave_max4(qd);   // zeros where the lane has no node
         if ((t & 63) < 4) S.sRes[t >> 6][t & 3] = m;
@@ -1068,7 +1068,10 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (a.do_resid && t < 4) {
         uint64_t v = S.sRes[0][t];
         for (int w = 1; w < TPB / 64; ++w) v = max(v, S.sRes[w][t]);
-        a.resid_part[rslot * 4 + wave_max4_value(t)] = __longlong_as_double((long long)v);
+        const int c = wave_max4_value(t);
+        // few workgroups: straight into the handle's four maxima, cleared by the step's first stage
+        if (a.resid_max) atomicMax((unsigned long long *)(a.resid_max + c * kResidStride), (unsigned long long)v);
+        else a.resid_part[rslot * 4 + c] = __longlong_as_double((long long)v);
     }
     if (a.mode == 0) {
         R qn[4];   // the next stage's own Q trace in the compute type (IP epilogue)
@@ -1134,6 +1137,7 @@ __global__ __launch_bounds__((Tile<P, EPB>::TPB)) void k_stage(StageArgs a) {
         if (a.dt_cg) cg *= d;
     }
     const int b = xcd_tile(blockIdx.x, gridDim.x);
+    if (a.resid_max && !a.do_resid && b == 0 && threadIdx.x < 4) a.resid_max[threadIdx.x * kResidStride] = 0.0;
     stage_body<P, EPB, NS, IP, RS, R, TR, XBF>(a, b * EPB, b, cq, cg, S);
 }
 
