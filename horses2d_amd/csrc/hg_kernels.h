@@ -1157,9 +1157,16 @@ __global__ __launch_bounds__(256) void k_dt_elem(const double *Q, int K, double 
     }
     su[t] = u; sa[t] = aa;
     __syncthreads();
-    if (t < EPB * PP && e < K && n == 0) {
+    // P lanes each a column's maximum, then one lane theirs (2 P dependent reads instead of P^2)
+    const bool col = t < EPB * PP && e < K && n < P;
+    if (col) {
+        for (int x = n + P; x < PP; x += P) { u = fmax(u, su[s * PP + x]); aa = fmax(aa, sa[s * PP + x]); }
+        su[t] = u; sa[t] = aa;   // entries below P, which no lane reads above
+    }
+    __syncthreads();
+    if (col && n == 0) {
         double mu = 0.0, ma = 0.0;
-        for (int x = 0; x < PP; ++x) { mu = fmax(mu, su[s * PP + x]); ma = fmax(ma, sa[s * PP + x]); }
+        for (int x = 0; x < P; ++x) { mu = fmax(mu, su[s * PP + x]); ma = fmax(ma, sa[s * PP + x]); }
         umax[e] = mu; amax[e] = ma;
     }
 }
