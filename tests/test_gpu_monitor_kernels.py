@@ -1,9 +1,11 @@
 """The reductions behind the monitors at the edges of their rounds: the time-step scan (4096 elements
 a round), the conservation sums (1024 partials a round), the probes at the smallest and largest order.
 
-The scan's maxima and minimum are exact in any order, so it is compared with numpy's prefix maxima at
-1e-15 (the last division); the sums at 1e-13 of the sum of magnitudes (sqrt of the term count times
-the unit rounding), the probes at 1e-14 of the state (at most 13 products a coordinate)."""
+The scan's maxima and minimum are exact in any order; numpy's prefix maxima take the element side from
+the mesh's extent, while the library subtracts corner coordinates (rounded at 5, over sides down to
+0.04: 1e-13), hence 1e-12.  The sums are compared at 1e-13 of the sum of magnitudes (the unit rounding
+times the depth of the additions), the probes at 1e-13 of the state (two interpolations of at most 13
+products with weights below 4)."""
 import numpy as np
 import pytest
 
@@ -25,15 +27,15 @@ def test_scan_and_sums(nx, ny, N):
     K, P = nx * ny, N + 1
     rng = np.random.Generator(np.random.PCG64(K))
     Q = dg.state().reshape(K, P * P, 4)
-    Q *= 1.0 + 0.3 * rng.uniform(size=(K, 1, 1))        # uneven elements: the running maxima matter
+    Q[..., 3] *= 1.0 + 0.3 * rng.uniform(size=(K, 1))   # uneven elements: the running maxima matter
     dg.upload(Q.reshape(-1))
     u = np.hypot(Q[..., 1], Q[..., 2]) / Q[..., 0]
     a = np.sqrt(1.4 * 0.4 * (Q[..., 3] / Q[..., 0] - 0.5 * u * u))
     um, am = np.maximum.accumulate(u.max(1)), np.maximum.accumulate(a.max(1))
     dt = np.min(0.5 * np.sqrt(1.4) * 0.1 * min(10.0 / nx, 10.0 / ny) / (um + am) / P)
-    assert dg.estimate_dt(1e30, 0.1) == pytest.approx(dt, rel=1e-13)
+    assert dg.estimate_dt(1e30, 0.1) == pytest.approx(dt, rel=1e-12)
     again = np.min(0.5 * np.sqrt(1.4) * 0.1 * min(10.0 / nx, 10.0 / ny) / (um[-1] + am[-1]) / P)
-    assert dg.estimate_dt(1e30, 0.1) == pytest.approx(again, rel=1e-13)   # the saved maxima
+    assert dg.estimate_dt(1e30, 0.1) == pytest.approx(again, rel=1e-12)   # the saved maxima
     w = 0.5 * np.polynomial.legendre.leggauss(P)[1]
     terms = Q * (np.outer(w, w).reshape(-1) * (100.0 / K))[None, :, None]
     got = dg.conservation_sums()
@@ -55,4 +57,4 @@ def test_probes_on_nodes_and_between(N):
         return c / c.sum()
     dg.probes_set(el, xi, eta, [("rho", "rhou", "rhov", "rhoe")[k % 4] for k in range(70)])
     ref = np.array([lag(eta[k]) @ Q[el[k], :, :, k % 4] @ lag(xi[k]) for k in range(70)])
-    assert np.max(np.abs(dg.probes_update() - ref)) <= 1e-14 * np.max(np.abs(Q)) * P
+    assert np.max(np.abs(dg.probes_update() - ref)) <= 1e-13 * np.max(np.abs(Q))
