@@ -87,7 +87,7 @@ __device__ __forceinline__ int xcd_tile(int b, int nb) {
 template <int P>
 struct Layout {
     static constexpr int RS = P + ((P == 4 || P == 8) ? 1 : 0);
-    static constexpr int ES = P * RS + ((P == 3 || P == 6) ? 3 : P == 7 ? 7 : 0);
+    static constexpr int ES = P * RS + ((P == 3 || P == 6) ? 3 : P == 7 ? 7 : P == 8 ? -1 : 0);
     // entry of node n (= i + P j) of the tile's element s
     __device__ static constexpr int at(int s, int n) { return s * ES + n + (RS - P) * (n / P); }
 };
@@ -142,7 +142,7 @@ struct Quads {
 // fma in l order so that every kernel that forms a trace (prolongation, stage epilogue) produces
 // the same bits; A = T accumulates in the tile's own type (the FP32 form's gradient traces, which
 // only the kernel that forms them ever evaluates).
-template <int P, int NL, typename T, typename A>
+template <int P, int NL, int UNROLL = P, typename T, typename A>
 __device__ __forceinline__ void face_trace(const T *X, int x0, const A *sLb, int f, int k, A *out) {
     const A *lb = (f == 0 || f == 3) ? sLb : sLb + P;
     // nodes (k, l) of a horizontal face or (l, k) of a vertical one: a base and a stride, so
@@ -152,8 +152,7 @@ __device__ __forceinline__ void face_trace(const T *X, int x0, const A *sLb, int
     const int base = x0 + (horiz ? k : RS * k), step = horiz ? RS : 1;
 #pragma unroll
     for (int c = 0; c < 4; ++c) out[c] = A(0);
-    // a rolled loop keeps one node's values live (unrolled, all P nodes are loaded up front)
-#pragma unroll 1
+#pragma unroll UNROLL
     for (int l = 0; l < P; ++l) {
         T v[4];
         Quads<T, NL>::get(X, base + step * l, v);
@@ -163,7 +162,7 @@ __device__ __forceinline__ void face_trace(const T *X, int x0, const A *sLb, int
 }
 
 // The same for an eight-value array (two Quads arrays one after the other): one pass over the nodes.
-template <int P, int NL, typename T, typename A>
+template <int P, int NL, int UNROLL = P, typename T, typename A>
 __device__ __forceinline__ void face_trace8(const T *X, int x0, const A *sLb, int f, int k, A *out) {
     const A *lb = (f == 0 || f == 3) ? sLb : sLb + P;
     constexpr int RS = Layout<P>::RS;
@@ -171,7 +170,7 @@ __device__ __forceinline__ void face_trace8(const T *X, int x0, const A *sLb, in
     const int base = x0 + (horiz ? k : RS * k), step = horiz ? RS : 1;
 #pragma unroll
     for (int c = 0; c < 8; ++c) out[c] = A(0);
-#pragma unroll 1
+#pragma unroll UNROLL
     for (int l = 0; l < P; ++l) {
         T v[8];
         Quads<T, NL>::get(X, base + step * l, v);
@@ -300,19 +299,17 @@ __device__ __forceinline__ void br1_face_flux(const StageArgs &a, const Phys<R> 
 // q: the tile's state in the compute type (Quads; energy slot shifted in the FP32 form), Ja: its
 // metric (Quads: Ja11, Ja21, Ja12, Ja22), x0 the element's first entry in both, Fu: element uStar
 // fluxes [(f*P + k)*6] (see br1_face_flux), sHat: hatD transposed (hatD(i, l) at [l*P + i]).
-// ROLLED keeps the two l loops rolled (one node's values live; the stage kernel, where the
-// registers bound occupancy); the sums are the same either way.
 // Faces whose bit 8 + f is set in ord are curved p-non-conforming or subdivided edges, whose
 // lift terms come per direction from the mortar kernel (uStar dS n projected direction by
 // direction): the face lane stores the x terms with the "normal" (1, 0), and mortar_y_lift adds
 // the y terms afterwards.
-template <int P, int NL, typename R, bool ROLLED = false>
+template <int P, int NL, typename R, int UNROLL = P>
 __device__ __forceinline__ void br1_node_gradient(const R *q, const R *Ja, int x0, const R *sHat, const R *Fu,
                                                   const R *sLbw, int ord, int i, int j, R ijac, R *dq) {
     // Every accumulator receives its xi terms (l = 0..P-1) then its eta terms; each state value
     // is read once and used for both directions, and the metric-weighted derivative entry
     // Ja * hatD is formed once per node for all four variables.
-    constexpr int UNROLL = ROLLED ? 1 : P, RS = Layout<P>::RS;
+    constexpr int RS = Layout<P>::RS;
     using V = Quads<R, NL>;
     R acc[8];
 #pragma unroll
@@ -383,12 +380,12 @@ __device__ __forceinline__ void mortar_y_lift(const double *mu8, const R *sLbw, 
 
 // Interior (broken) gradient of the IP method (QuadElement_QuadProcedures.incf:42-88); q as above.
 // sD: D transposed (D(i, l) at [l*P + i]).
-template <int P, int NL, typename R>
+template <int P, int NL, typename R, int UNROLL = P>
 __device__ __forceinline__ void ip_node_gradient(const R *q, int x0, const R *sD, int i, int j, R j11, R j12, R j21,
                                                  R j22, R ijac, R *dq) {
-    // l outermost (each accumulator still sums l = 0..P-1 in order): one node's values live
+    // l outermost (each accumulator still sums l = 0..P-1 in order): few nodes' values live
     R dxi[4] = {R(0), R(0), R(0), R(0)}, deta[4] = {R(0), R(0), R(0), R(0)};
-#pragma unroll 1
+#pragma unroll UNROLL
     for (int l = 0; l < P; ++l) {
         const R di = sD[l * P + i], dj = sD[l * P + j];
         R qx[4], qy[4];
@@ -497,15 +494,15 @@ __device__ __forceinline__ void stored_trace(const StageArgs &a, int fe, int ff,
 // walls :279-318).  The gradient trace is accumulated in FP64 in the FP64 form and in FP32 in
 // the FP32 form (lbR: lb in the compute type).
 // mdq: where a p-non-conforming face keeps its gradient trace for the mortar kernel (or null).
-template <int P, int NL, typename R, typename TR>
+template <int P, int NL, typename R, typename TR, int UNROLL = P>
 __device__ __forceinline__ void viscous_face_trace(const StageArgs &a, const Phys<R> &ph, int flags, const R *qs,
                                                    const R *sDQ, int x0, const double *sLb, const R *lbR, int ff,
                                                    int fk, TR *o, R muf, double *mdq = nullptr) {
     R ds[8], fv[4], gv[4];
     if constexpr (sizeof(R) == 4) {
-        face_trace8<P, NL>(sDQ, x0, lbR, ff, fk, ds);
+        face_trace8<P, NL, UNROLL>(sDQ, x0, lbR, ff, fk, ds);
     } else {
-        face_trace8<P, NL>(sDQ, x0, sLb, ff, fk, ds);
+        face_trace8<P, NL, UNROLL>(sDQ, x0, sLb, ff, fk, ds);
     }
     if (mdq) {
 #pragma unroll
@@ -632,7 +629,6 @@ struct StageSmem {
     using T = Tile<P, EPB>;
     alignas(16) double sQ[T::NL * 4];
     alignas(16) double sLb[2 * P];
-    alignas(16) uint64_t sRes[4][4];
     struct Fluxes {
         alignas(16) R sCF[T::NL * 4];          // BR1: the metric Ja during the gradient phase
         alignas(16) R sCG[T::NL * 4];          // NS, FP32: the compute-type state until the node phase
@@ -642,17 +638,25 @@ struct StageSmem {
         Fluxes f;
         alignas(16) R sDQ[IP ? T::NL * 8 : 1];
     } u;
-    alignas(16) R sF[NS && !IP ? T::NF * 6 : T::NF * 4];  // BR1: uStar fluxes during the gradient phase
+    // the face fluxes (BR1: uStar fluxes during the gradient phase); once every wavefront has
+    // lifted them, the residual maxima
+    union {
+        alignas(16) R sF[NS && !IP ? T::NF * 6 : T::NF * 4];
+        uint64_t sRes[4][4];
+    };
     // IP gradient-face terms: the face phase's contravariant fluxes, then (same arrays) the
     // U / V lift coefficients
     alignas(16) R sU[IP ? T::NF * 4 : 1];
     alignas(16) R sV[IP ? T::NF * 4 : 1];
     alignas(16) R sHat[T::PP];          // transposed, as sD: a wavefront's reads are consecutive
     alignas(16) R sD[NS ? T::PP : 1];   // IP gradient; BR1: the Laplacian dissipation's interior gradient
-    alignas(16) R sLbw[2 * P];
+    alignas(16) R sLbw[IP && sizeof(R) == 4 ? 4 * P : 2 * P];   // lbw; IP in FP32: lb (epilogue) behind it
     alignas(16) R sDlbw[2 * P];
-    alignas(16) R sLbR[IP ? 2 * P : 1];   // lb in the compute type (IP epilogue, FP32 traces)
 };
+
+// Wavefronts per SIMD the stage kernel's register allocation has to leave room for: four of the FP64
+// Navier-Stokes form with one solver (P = 8, interior penalty: 129 registers without it).
+constexpr int stage_waves(bool ns, bool one_solver, bool fp64) { return ns && one_solver && fp64 ? 4 : 1; }
 
 // One element tile [e0, e0+EPB) of a stage; any workgroup size >= Tile<P, EPB>::TPB (at most
 // 256).  rslot is the residual partial this tile writes; cq, cg are the stage's RK factors.
@@ -671,6 +675,11 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     constexpr bool XB = RS < 0 || XBF;
     constexpr int PP = T::PP, NN = T::NN, NF = T::NF;
     constexpr bool BR1 = NS && !IP;
+    // The contraction and trace loops, whose sums are the same either way.  Unrolled, their LDS reads
+    // overlap (2 to 5 % of a step at every order); the kernels with every solver or boundary kind
+    // compiled in, and FP32 interior penalty, are where the registers this takes cost a wavefront per SIMD
+    // (256 x 256, N = 7, mixed: 78 registers and 543 us a step at 2, 81 and 575 us unrolled).
+    constexpr int UNROLL = XB ? 1 : (IP && sizeof(R) == 4) ? 2 : P;
     const int TPB = blockDim.x;
     double *sQ = S.sQ, *sLb = S.sLb;
     R *sCF = S.u.f.sCF, *sCG = S.u.f.sCG, *sF = S.sF, *sU = S.sU, *sV = S.sV;
@@ -680,7 +689,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     const bool ipgrad = IP && a.ph.ip_gradflux;
     if (t < 2 * P) {
         sLb[t] = a.lb[t]; sLbw[t] = (R)a.lbw[t]; sDlbw[t] = (R)a.dlbw[t];
-        if (IP) S.sLbR[t] = (R)a.lb[t];
+        if (IP && sizeof(R) == 4) sLbw[2 * P + t] = (R)a.lb[t];
     }
     for (int x = t; x < PP; x += TPB) {
         const int xt = (x % P) * P + x / P;
@@ -743,11 +752,11 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (NS && node_active) {
         const int i = n % P, j = n / P;
         if (BR1) {
-            br1_node_gradient<P, NL, R, true>(sQr, sCF, x0, sHat, sF + s * 4 * P * 6, sLbw, ord, i, j, ijac, dq);
+            br1_node_gradient<P, NL, R, UNROLL>(sQr, sCF, x0, sHat, sF + s * 4 * P * 6, sLbw, ord, i, j, ijac, dq);
             if (ord >> 8) mortar_y_lift<P, R>(a.mustar + (int64_t)e * 4 * P * 8, sLbw, ord, i, j, ijac, dq);
         }
-        else ip_node_gradient<P, NL, R>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dq);
-        if (LAPG && a.lap) ip_node_gradient<P, NL, R>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dqi);
+        else ip_node_gradient<P, NL, R, UNROLL>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dq);
+        if (LAPG && a.lap) ip_node_gradient<P, NL, R, UNROLL>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dqi);
     }
     // the neighbour's viscous flux trace, issued before the barrier and consumed in the face phase
     R vn[NS ? VT : 1];
@@ -997,7 +1006,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (node_active) {
         const int i = n % P, j = n / P;
         R acc[4] = {R(0), R(0), R(0), R(0)};
-#pragma unroll 1
+#pragma unroll UNROLL
         for (int l = 0; l < P; ++l) {
             const R hi = sHat[l * P + i], hj = sHat[l * P + j];
             R cF[4], cG[4];
@@ -1058,13 +1067,14 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             Quads<double, NL>::put(sQ, xn, qn);
         }
     }
-    // max|QDot| per equation: across the wavefront here, across the workgroup's wavefronts after the
-    // barrier; one partial per workgroup (reduced by k_resid_final), or one atomic maximum
+    __syncthreads();
+    // max|QDot| per equation: across the wavefront, then across the workgroup's wavefronts; one
+    // partial per workgroup (reduced by k_resid_final), or one atomic maximum
     if (a.do_resid) {
         const uint64_t m = wave_max4(qd);   // zeros where the lane has no node
         if ((t & 63) < 4) S.sRes[t >> 6][t & 3] = m;
+        __syncthreads();
     }
-    if (a.do_resid || a.mode == 0) __syncthreads();
     if (a.do_resid && t < 4) {
         uint64_t v = S.sRes[0][t];
         for (int w = 1; w < TPB / 64; ++w) v = max(v, S.sRes[w][t]);
@@ -1077,7 +1087,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         R qn[4];   // the next stage's own Q trace in the compute type (IP epilogue)
         if (face_active) {
             double tq[4];
-            face_trace<P, NL>(sQ, fs * Layout<P>::ES, sLb, ff, fk, tq);
+            face_trace<P, NL, UNROLL>(sQ, fs * Layout<P>::ES, sLb, ff, fk, tq);
             tq[3] = slot_energy<TR>(a.ph, tq[3]);
             TR *o = (TR *)a.tr_out + ((int64_t)(fe * 4 + ff) * P + fk) * 4;
 #pragma unroll
@@ -1108,7 +1118,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                 // FP64 kernel a wavefront per SIMD
                 R m11, m12, m21, m22, mij;
                 load_metric<P, R>(a, e, n, g, m11, m12, m21, m22, mij);
-                ip_node_gradient<P, NL, R>(sQn, x0, sD, n % P, n / P, m11, m12, m21, m22, mij, dq);
+                ip_node_gradient<P, NL, R, UNROLL>(sQn, x0, sD, n % P, n / P, m11, m12, m21, m22, mij, dq);
             }
             __syncthreads();   // the state copy and the fluxes' space are free
             R *sDQ = S.u.sDQ;
@@ -1119,7 +1129,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             __syncthreads();
             if (face_active) {
                 double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + ((int64_t)(fe * 4 + ff) * P + fk) * 8 : nullptr;
-                viscous_face_trace<P, NL, R, TR>(a, ph, fr.x, qn, sDQ, fs * Layout<P>::ES, sLb, S.sLbR, ff, fk,
+                viscous_face_trace<P, NL, R, TR, UNROLL>(a, ph, fr.x, qn, sDQ, fs * Layout<P>::ES, sLb, sLbw + 2 * P, ff, fk,
                                                 (TR *)a.dtr_out + ((int64_t)(fe * 4 + ff) * P + fk) * VT, ph.mu, mdq);
             }
           }
@@ -1128,7 +1138,8 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
 }
 
 template <int P, int EPB, bool NS, bool IP, int RS, typename R, typename TR, bool XBF = false>
-__global__ __launch_bounds__((Tile<P, EPB>::TPB)) void k_stage(StageArgs a) {
+__global__ __launch_bounds__((Tile<P, EPB>::TPB))
+    __attribute__((amdgpu_waves_per_eu(stage_waves(NS, RS >= 0 && !XBF, sizeof(R) == 8)))) void k_stage(StageArgs a) {
     __shared__ StageSmem<P, EPB, NS, IP, R> S;
     double cq = a.cq, cg = a.cg;
     if (a.dt_dev) {   // graph replay: the step size lives in device memory
