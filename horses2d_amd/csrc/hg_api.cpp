@@ -5,6 +5,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -989,6 +990,8 @@ int hg_create(const hg_mesh_desc *mesh, const hg_physics *phys, const hg_options
         std::iota(all.begin(), all.end(), 0);
         if (setup_handle(h.get(), m, phys, opt, all, all, mort)) return 1;
     }
+    h->pool_open = true;
+    hg::transfers_open();
     *out = h.release();
     return 0;
 }
@@ -996,6 +999,7 @@ int hg_create(const hg_mesh_desc *mesh, const hg_physics *phys, const hg_options
 int hg_destroy(hg_handle *h) {
     if (!h) return 0;
     if (h->stream) hipStreamSynchronize(h->stream);
+    if (h->pool_open) hg::transfers_close();
     for (auto *s : h->sub) {
         s->stream = nullptr;   // shared with this handle
         hg_destroy(s);
@@ -1089,12 +1093,23 @@ int hg_build_geometry(const hg_mesh_desc *mesh, int64_t nnodes, double *X, doubl
     return 0;
 }
 
-// The mean nodal pressure of a state (0 when it is not finite).
+// The mean nodal pressure of a state (0 when it is not finite).  The divisions are shared out, the
+// sum runs over the nodes in order: the FP32 form's rounding follows every bit of this value.
 static double mean_pressure(double gm1, const double *Q, int64_t nodes) {
-    double sum = 0.0;
-    for (int64_t n = 0; n < nodes; ++n) {
+    auto pressure = [&](int64_t n) {
         const double *q = Q + 4 * n;
-        sum += gm1 * (q[3] - 0.5 * (q[1] * q[1] + q[2] * q[2]) / q[0]);
+        return gm1 * (q[3] - 0.5 * (q[1] * q[1] + q[2] * q[2]) / q[0]);
+    };
+    double sum = 0.0;
+    try {
+        std::vector<double> p(nodes);
+        hg::in_shares(nodes, 65536, [&](int64_t n0, int64_t n1) {
+            for (int64_t n = n0; n < n1; ++n) p[n] = pressure(n);
+        });
+        for (double v : p) sum += v;
+    } catch (const std::exception &) {   // no memory for them
+        sum = 0.0;
+        for (int64_t n = 0; n < nodes; ++n) sum += pressure(n);
     }
     const double pref = nodes > 0 ? sum / (double)nodes : 0.0;
     return std::isfinite(pref) ? pref : 0.0;
@@ -1136,7 +1151,7 @@ int hg_upload_state(hg_handle *h, const double *Q, int64_t ndof) {
     // the captured kernels carry the physics parameters (the FP32 form's reference pressure)
     // by value: recapture only if it changed
     if (h->ph.pref != pref_old) drop_graphs(h);
-    HG_CHECK(hipMemcpyAsync(h->Q, Q, ndof * sizeof(double), hipMemcpyHostToDevice, h->stream));
+    HG_CHECK(hg::copy_to_device(h, h->Q, Q, ndof * sizeof(double)));
     hg::StageArgs a = base_args(h);
     h->cur = 0;
     a.tr_out = h->tr[0];
@@ -1144,7 +1159,6 @@ int hg_upload_state(hg_handle *h, const double *Q, int64_t ndof) {
     h->vtr_valid = false;
     h->qdot_valid = false;
     h->mon_tr = -1;
-    HG_CHECK(hipStreamSynchronize(h->stream));
     return 0;
 }
 
@@ -1165,8 +1179,7 @@ int hg_download_state(hg_handle *h, double *Q, int64_t ndof) {
     if (!h || !Q) return set_err("hg_download_state: null argument");
     if (ndof != h->ndof) return set_err("hg_download_state: ndof mismatch");
     if (!h->sub.empty()) return composite_gather(h, false, Q);
-    HG_CHECK(hipMemcpyAsync(Q, h->Q, ndof * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::copy_to_host(h, Q, h->Q, ndof * sizeof(double)));
     return 0;
 }
 
@@ -1174,8 +1187,7 @@ int hg_download_qdot(hg_handle *h, double *QDot, int64_t ndof) {
     if (!h || !QDot) return set_err("hg_download_qdot: null argument");
     if (ndof != h->ndof) return set_err("hg_download_qdot: ndof mismatch");
     if (!h->sub.empty()) return composite_gather(h, true, QDot);
-    HG_CHECK(hipMemcpyAsync(QDot, h->QDot, ndof * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::copy_to_host(h, QDot, h->QDot, ndof * sizeof(double)));
     return 0;
 }
 
@@ -1248,10 +1260,7 @@ int hg_residuals(hg_handle *h, double res[4]) {
         }
         return 0;
     }
-    double r[3 * hg::kResidStride + 1];
-    HG_CHECK(hipMemcpyAsync(r, h->resid, sizeof(r), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
-    for (int c = 0; c < 4; ++c) res[c] = r[c * hg::kResidStride];
+    HG_CHECK(hg::read_values(h, res, h->resid, 4, hg::kResidStride));
     return 0;
 }
 
@@ -1273,8 +1282,7 @@ int hg_estimate_dt(hg_handle *h, double dt_max, double cfl, double *dt) {
         HG_CHECK(hg::launch_dt_scan(h->K, h->umax, h->amax, h->dx, coef, (double)(h->N + 1), dt_max, h->dtstate,
                                     h->dtout, h->stream));
     }
-    HG_CHECK(hipMemcpyAsync(dt, h->dtout, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::read_values(h, dt, h->dtout, 1));
     return 0;
 }
 
@@ -1297,8 +1305,7 @@ int hg_conservation_sums(hg_handle *h, double out[4]) {
         return 0;
     }
     HG_CHECK(hg::launch_cons_sums(h->P, h->Q, h->jac64, h->w, h->K, h->cons_partial, h->cons_nb, h->cons_out, h->stream));
-    HG_CHECK(hipMemcpyAsync(out, h->cons_out, 4 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::read_values(h, out, h->cons_out, 4));
     return 0;
 }
 
@@ -1319,8 +1326,7 @@ int hg_volume_integrals(hg_handle *h, double out[2]) {
     HG_CHECK(hg::launch_volume_integrals(h->P, h->Q, h->jac64, h->w, h->K, h->ph.gamma, h->ph.gm1, h->cons_partial,
                                          h->cons_nb, h->monitor_out, h->stream));
     double v[4];
-    HG_CHECK(hipMemcpyAsync(v, h->monitor_out, 4 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::read_values(h, v, h->monitor_out, 4));
     out[0] = v[0];
     out[1] = std::sqrt(v[1]);
     return 0;
@@ -1469,8 +1475,7 @@ int hg_surface_integrals(hg_handle *h, int32_t marker, double out[9]) {
                                               h->stream));
     else
         HG_CHECK(hipMemsetAsync(h->monitor_out, 0, 9 * sizeof(double), h->stream));
-    HG_CHECK(hipMemcpyAsync(out, h->monitor_out, 9 * sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::read_values(h, out, h->monitor_out, 9));
     return 0;
 }
 
@@ -1559,8 +1564,7 @@ int hg_probes_update(hg_handle *h, double *out) {
                            "last step or upload");
     HG_CHECK(hg::launch_probes(h->Q, h->QDot, h->probe_ev, h->probe_l, h->nprobes, h->P, h->ph.gm1, h->ph.gamma,
                                h->probe_out, h->stream));
-    HG_CHECK(hipMemcpyAsync(out, h->probe_out, sizeof(double) * h->nprobes, hipMemcpyDeviceToHost, h->stream));
-    HG_CHECK(hipStreamSynchronize(h->stream));
+    HG_CHECK(hg::read_values(h, out, h->probe_out, h->nprobes));
     return 0;
 }
 

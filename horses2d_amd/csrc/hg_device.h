@@ -247,6 +247,10 @@ hipError_t launch_surface_integrals(bool mixed, const int *slots, int nslots, in
 // Jumps-based artificial viscosity per element from the stage's Q traces (and boundary states).
 hipError_t launch_art_visc(int P, bool mixed, const StageArgs &a, const double *evol, const double *w, double *mu_a,
                            hipStream_t st);
+// bytes (a multiple of 16) from src to dst, either of them pinned host memory.
+hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t st);
+// dst[i] = src[i * stride], i < n: a few values into pinned host memory.
+hipError_t launch_store_values(const double *src, int n, int stride, double *dst, hipStream_t st);
 // Probe values (Probe_Update): n probes, per probe an int2 (element, variable) and 2P
 // interpolant values; variables 4..7 read QDot, the others Q.
 hipError_t launch_probes(const double *Q, const double *QDot, const int2 *ev, const double *l, int n, int P,

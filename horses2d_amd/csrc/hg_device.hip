@@ -237,6 +237,15 @@ __global__ __launch_bounds__(64) void k_probes(const double *Q, const double *QD
     out[k] = o;
 }
 
+__global__ __launch_bounds__(256) void k_copy(const double2 *src, double2 *dst, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+__global__ __launch_bounds__(256) void k_store_values(const double *src, int n, int stride, double *dst) {
+    for (int i = threadIdx.x; i < n; i += 256) dst[i] = src[(int64_t)i * stride];
+}
+
 // Residual of each case of a batch (one workgroup): the maxima of its tiles' partials.
 __global__ __launch_bounds__(1024) void k_batch_resid(const double *part, const int2 *ranges, double *const *out) {
     const int2 r = ranges[blockIdx.x];
@@ -439,6 +448,17 @@ hipError_t launch_surface_integrals(bool mixed, const int *slots, int nslots, in
     else
         hipLaunchKernelGGL((k_surface_integrals<double>), dim3(1), dim3(1024), 0, st, slots, nslots, P,
                            (const double *)tr, (const double *)vtr, face, egeo, w, gm1, Eref, mu_a, mu, out);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy(const void *src, void *dst, size_t bytes, hipStream_t st) {
+    const int n = (int)(bytes / 16);
+    hipLaunchKernelGGL(k_copy, dim3((n + 255) / 256), dim3(256), 0, st, (const double2 *)src, (double2 *)dst, n);
+    return hipGetLastError();
+}
+
+hipError_t launch_store_values(const double *src, int n, int stride, double *dst, hipStream_t st) {
+    hipLaunchKernelGGL(k_store_values, dim3(1), dim3(256), 0, st, src, n, stride, dst);
     return hipGetLastError();
 }
 

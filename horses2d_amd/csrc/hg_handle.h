@@ -4,6 +4,7 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <functional>
 #include <string>
 #include <utility>
 #include <vector>
@@ -97,6 +98,7 @@ struct hg_handle {
     int nsubedge = 0;
     double *n1e = nullptr;                   // per mesh element: N + 1 (time-step scan)
     std::vector<std::vector<int>> sub_probes;   // per sub-handle: the probe indices it holds
+    bool pool_open = false;                  // this handle counts among the staging pool's users
     bool shared_stream = false;              // a sub-handle: the stream belongs to its parent
     int cur = 0;
     int tile[2] = {-1, -1};  // workgroup tile of the stage and gradient kernels, -1 = not chosen yet
@@ -144,6 +146,17 @@ int ensure_vtr(hg_handle *h);
 void mark_last_evaluation(hg_handle *h, int tr);
 // Records the message returned by hg_last_error and returns 1.
 int handle_error(const std::string &m);
+// Transfers through the process-wide pinned staging pool (hg_transfer.cpp), on the handle's stream.
+// copy_to_host returns with dst filled; copy_to_device with src free to change (the copy itself is
+// ordered on the stream).  read_values waits for the stream and returns src[i * stride], i < n.
+// Every handle opens the pool once and closes it when destroyed.
+hipError_t copy_to_host(hg_handle *h, void *dst, const void *src, size_t bytes);
+hipError_t copy_to_device(hg_handle *h, void *dst, const void *src, size_t bytes);
+hipError_t read_values(hg_handle *h, double *dst, const double *src, int n, int stride = 1);
+// f(first, last) over [0, n) in contiguous shares of at least `least`, on up to four threads.
+void in_shares(int64_t n, int64_t least, const std::function<void(int64_t, int64_t)> &f);
+void transfers_open();
+void transfers_close();
 // Locates the allocation-free entry points' scratch array on a device (once per device).
 int noalloc_setup(int device);
 }  // namespace hg

@@ -264,12 +264,12 @@ class DGSEM:
         _check(self._L.hg_upload_state(self._h, _ptr(Q), Q.size), "hg_upload_state")
 
     def state(self) -> np.ndarray:
-        Q = np.zeros(self.ndof)
+        Q = np.empty(self.ndof)
         _check(self._L.hg_download_state(self._h, _ptr(Q), self.ndof), "hg_download_state")
         return Q
 
     def qdot(self) -> np.ndarray:
-        Q = np.zeros(self.ndof)
+        Q = np.empty(self.ndof)
         _check(self._L.hg_download_qdot(self._h, _ptr(Q), self.ndof), "hg_download_qdot")
         return Q
 
