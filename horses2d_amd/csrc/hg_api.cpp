@@ -367,16 +367,102 @@ int composite_stage(hg_handle *h, double am, double cq, double cg, bool first, b
     return 0;
 }
 
+// The tables of the one-launch passes, from the sub-handles' current buffers and physics (every change
+// of those drops the captured graphs, and this runs before a capture).
+int build_one_launch(hg_handle *h, const StepCoefs &k) {
+    const int ns = (int)h->sub.size();
+    h->ctile = h->sub.back()->tile[0] == 0 ? 0 : 1;
+    std::vector<int4> items;
+    std::vector<int2> ranges;
+    std::vector<double *> resid;
+    int most = 0;
+    h->cblock = 64;
+    for (int g = 0; g < ns; ++g) {
+        hg_handle *s = h->sub[g];
+        const int epb = hg::tile_elems(s->P, h->ctile), first = (int)items.size();
+        h->cblock = std::max(h->cblock, hg::tile_threads(s->P, h->ctile));
+        for (int e0 = 0; e0 < s->K; e0 += epb) items.push_back(make_int4(g, e0, s->P, (int)items.size()));
+        ranges.push_back(make_int2(first, (int)items.size()));
+        resid.push_back(s->resid);
+        most = std::max(most, (int)items.size() - first);
+    }
+    h->cnitems = (int)items.size();
+    h->catomic = k.nst > 1 && most <= hg::kResidAtomic;
+    std::vector<int> sched(items.size());
+    std::iota(sched.begin(), sched.end(), 0);
+    std::vector<hg::StageArgs> slots;
+    for (int g = 0; g < ns; ++g)
+        for (int p = 0; p < 2; ++p)
+            for (int st = 0; st < k.nst; ++st) {
+                hg_handle *s = h->sub[g];
+                hg::StageArgs a = base_args(s);
+                const int in = p ^ (st & 1);
+                a.tr_in = s->tr[in];
+                a.tr_out = s->tr[in ^ 1];
+                a.dtr = s->dtr[s->ip_fused ? in : 0];
+                a.dtr_out = s->dtr[s->ip_fused ? (in ^ 1) : 0];
+                a.am = k.am[st];
+                a.cq = k.cq[st];
+                a.cg = k.cg[st];
+                a.first_stage = st == 0 ? 1 : 0;
+                a.do_resid = st == k.nst - 1 ? 1 : 0;
+                a.resid_part = h->cpart;
+                if (h->catomic && (st == 0 || a.do_resid)) a.resid_max = s->resid;
+                slots.push_back(a);
+            }
+    HG_CHECK(hipStreamSynchronize(h->stream));   // an earlier step may still read the old tables
+    HG_CHECK(hipMemcpy(h->citems, items.data(), items.size() * sizeof(int4), hipMemcpyHostToDevice));
+    HG_CHECK(hipMemcpy(h->csched, sched.data(), sched.size() * sizeof(int), hipMemcpyHostToDevice));
+    HG_CHECK(hipMemcpy(h->cranges, ranges.data(), ranges.size() * sizeof(int2), hipMemcpyHostToDevice));
+    HG_CHECK(hipMemcpy(h->cresid, resid.data(), resid.size() * sizeof(double *), hipMemcpyHostToDevice));
+    HG_CHECK(hipMemcpy(h->cslots, slots.data(), slots.size() * sizeof(hg::StageArgs), hipMemcpyHostToDevice));
+    return 0;
+}
+
+// composite_stage for the captured step of a handle with one_launch: the sub-handles' gradient passes
+// in one launch and their stages in one, the same bodies and so the same bits.
+int one_launch_stage(hg_handle *h, const StepCoefs &k, int parity, int st) {
+    const hg_handle *s0 = h->sub[0];
+    hg::BatchArgs b{};
+    b.slots = h->cslots;
+    b.nslots = 2 * k.nst;
+    b.slot = parity * k.nst + st;
+    b.items = h->citems;
+    b.sched = h->csched;
+    b.nitems = h->cnitems;
+    b.dt = h->dt_dev;
+    b.dt_cq = k.dt_cq;
+    b.dt_cg = k.dt_cg;
+    const int variant = 2 * (h->ph.ns ? (h->ph.viscous == HG_VISCOUS_IP ? 2 : 1) : 0) + (s0->mixed ? 1 : 0);
+    if (h->ph.ns) {
+        if (h->ph.viscous == HG_VISCOUS_BR1) {
+            HG_CHECK(hg::launch_mortar_ustar(mortar_args(h), h->stream));
+            HG_CHECK(hg::launch_sub_ustar(mortar_args(h), h->stream));
+        }
+        if (!s0->ip_fused) HG_CHECK(hg::launch_batch_gradient(variant, h->ctile, b, h->cblock, h->stream));
+    }
+    HG_CHECK(hg::launch_mortar_flux(mortar_args(h), h->stream));
+    HG_CHECK(hg::launch_sub_flux(mortar_args(h), h->stream));
+    HG_CHECK(hg::launch_batch_stage(variant, s0->ph.rs_kernel, h->ctile, b, h->cblock, h->stream));
+    if (st == k.nst - 1 && !h->catomic)
+        HG_CHECK(hg::launch_batch_resid(h->cpart, h->cranges, h->cresid, (int)h->sub.size(), h->stream));
+    h->cur ^= 1;
+    for (auto *s : h->sub) s->cur ^= 1;
+    return 0;
+}
+
 int build_composite_graphs(hg_handle *h, const StepCoefs &k) {
     const int cur0 = h->cur;
+    if (h->one_launch && build_one_launch(h, k)) return 1;
     for (int p = 0; p < 2; ++p) {
         h->cur = p;
         for (auto *s : h->sub) s->cur = p;
         HG_CHECK(hipStreamBeginCapture(h->stream, hipStreamCaptureModeThreadLocal));
         int bad = 0;
         for (int st = 0; st < k.nst && !bad; ++st)
-            bad = composite_stage(h, k.am[st], k.cq[st], k.cg[st], st == 0, st == k.nst - 1, 0, h->dt_dev, k.dt_cq,
-                                  k.dt_cg);
+            bad = h->one_launch ? one_launch_stage(h, k, p, st)
+                                : composite_stage(h, k.am[st], k.cq[st], k.cg[st], st == 0, st == k.nst - 1, 0,
+                                                  h->dt_dev, k.dt_cq, k.dt_cg);
         hipGraph_t g = nullptr;
         hipError_t e = hipStreamEndCapture(h->stream, &g);
         h->cur = cur0;
@@ -405,7 +491,8 @@ int composite_rk_step(hg_handle *h, double dt) {
         if (!h->dt_valid || dt != h->dt_last) {
             h->dt_last = dt;
             h->dt_valid = true;
-            HG_CHECK(hipMemcpyAsync(h->dt_dev, &h->dt_last, sizeof(double), hipMemcpyHostToDevice, h->stream));
+            for (double &d : h->dt_all) d = dt;
+            HG_CHECK(hipMemcpyAsync(h->dt_dev, h->dt_all, sizeof(h->dt_all), hipMemcpyHostToDevice, h->stream));
         }
         if (!h->gexec[0] && build_composite_graphs(h, k)) {
             drop_graphs(h);
@@ -936,8 +1023,21 @@ int create_composite(hg_handle *h, const hg_physics *phys, const hg_options *opt
     HG_CHECK(h->alloc(&h->amax, K));
     HG_CHECK(h->alloc(&h->dtstate, 2));
     HG_CHECK(h->alloc(&h->dtout, 1));
-    HG_CHECK(h->alloc(&h->dt_dev, 1));
+    HG_CHECK(h->alloc(&h->dt_dev, hg::kMaxSub));
     HG_CHECK(hipMemset(h->dtstate, 0, 2 * sizeof(double)));
+    // One launch per pass for all orders where the batched kernels hold them (points per direction up
+    // to 11) and the mesh's boundary kinds and solver are those of their one-solver forms.  The orders'
+    // launches of a stage otherwise run one after the other (60 x 48 elements of orders 4 and 6: 7.1
+    // and 7.6 us, of a 25 us stage).
+    h->one_launch = orders.size() > 1 && h->ph.rs_kernel >= 0 && !h->ph.xbc && orders.back() <= 10;
+    if (h->one_launch) {
+        HG_CHECK(h->alloc(&h->cslots, orders.size() * 10));
+        HG_CHECK(h->alloc(&h->citems, K));       // at least one element per tile
+        HG_CHECK(h->alloc(&h->csched, K));
+        HG_CHECK(h->alloc(&h->cpart, 4 * (size_t)K));
+        HG_CHECK(h->alloc(&h->cranges, orders.size()));
+        HG_CHECK(h->alloc(&h->cresid, orders.size()));
+    }
     HG_CHECK(hipDeviceSynchronize());
     return 0;
 }

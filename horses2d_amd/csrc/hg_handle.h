@@ -97,6 +97,18 @@ struct hg_handle {
     double *sgeo = nullptr;
     int nsubedge = 0;
     double *n1e = nullptr;                   // per mesh element: N + 1 (time-step scan)
+    // the captured step's passes over the element tiles of every order in one launch: a slot
+    // table of the sub-handles' arguments per trace parity and stage, the work list of their tiles
+    // (the batched kernels' form), the residual partials of each sub-handle and where they go
+    bool one_launch = false;
+    hg::StageArgs *cslots = nullptr;
+    int4 *citems = nullptr;
+    int *csched = nullptr;
+    int2 *cranges = nullptr;
+    double *cpart = nullptr, **cresid = nullptr;
+    int cnitems = 0, cblock = 0, ctile = 1;
+    bool catomic = false;
+    double dt_all[hg::kMaxSub] = {};         // dt_dev's content: the step size per sub-handle
     std::vector<std::vector<int>> sub_probes;   // per sub-handle: the probe indices it holds
     bool pool_open = false;                  // this handle counts among the staging pool's users
     bool shared_stream = false;              // a sub-handle: the stream belongs to its parent

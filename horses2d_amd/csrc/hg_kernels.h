@@ -679,7 +679,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     // overlap (2 to 5 % of a step at every order); the kernels with every solver or boundary kind
     // compiled in, and FP32 interior penalty, are where the registers this takes cost a wavefront per SIMD
     // (256 x 256, N = 7, mixed: 78 registers and 543 us a step at 2, 81 and 575 us unrolled).
-    constexpr int UNROLL = XB ? 1 : (IP && sizeof(R) == 4) ? 2 : P;
+    constexpr int UNROLL = (XB || RS == 2) ? 1 : (IP && sizeof(R) == 4) ? 2 : P;
     const int TPB = blockDim.x;
     double *sQ = S.sQ, *sLb = S.sLb;
     R *sCF = S.u.f.sCF, *sCG = S.u.f.sCG, *sF = S.sF, *sU = S.sU, *sV = S.sV;
@@ -687,6 +687,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     const int t = threadIdx.x;
     const Phys<R> ph(a.ph);
     const bool ipgrad = IP && a.ph.ip_gradflux;
+    if (a.resid_max && !a.do_resid && e0 == 0 && t < 4) a.resid_max[t * kResidStride] = 0.0;
     if (t < 2 * P) {
         sLb[t] = a.lb[t]; sLbw[t] = (R)a.lbw[t]; sDlbw[t] = (R)a.dlbw[t];
         if (IP && sizeof(R) == 4) sLbw[2 * P + t] = (R)a.lb[t];
@@ -1148,7 +1149,6 @@ __global__ __launch_bounds__((Tile<P, EPB>::TPB))
         if (a.dt_cg) cg *= d;
     }
     const int b = xcd_tile(blockIdx.x, gridDim.x);
-    if (a.resid_max && !a.do_resid && b == 0 && threadIdx.x < 4) a.resid_max[threadIdx.x * kResidStride] = 0.0;
     stage_body<P, EPB, NS, IP, RS, R, TR, XBF>(a, b * EPB, b, cq, cg, S);
 }
 
