@@ -87,6 +87,25 @@ bool line_metric(const std::vector<double> &metric, int K, int P, std::vector<do
     return true;
 }
 
+// Whether every element is a parallelogram to the mesh builder's rounding: each Ja component, a sum of
+// terms as large as the element's coordinates (reach: the largest of its corners'), spreads over its
+// lines by at most eight units in the last place of those.
+bool parallelograms(const std::vector<double> &lines, const std::vector<double> &reach, int K, int P) {
+    const size_t half = 2 * (size_t)K * P;
+    for (int e = 0; e < K; ++e) {
+        double lo[4], hi[4], scale = reach[e];   // Ja11, Ja21, Ja12, Ja22
+        for (int c = 0; c < 4; ++c) {
+            const double *L = &lines[(c / 2) * half + 2 * (size_t)e * P + c % 2];
+            lo[c] = hi[c] = L[0];
+            for (int k = 1; k < P; ++k) { lo[c] = std::fmin(lo[c], L[2 * k]); hi[c] = std::fmax(hi[c], L[2 * k]); }
+            scale = std::fmax(scale, std::fmax(std::fabs(lo[c]), std::fabs(hi[c])));
+        }
+        for (int c = 0; c < 4; ++c)
+            if (!(hi[c] - lo[c] <= std::ldexp(scale, -49))) return false;
+    }
+    return true;
+}
+
 hg::StageArgs base_args(hg_handle *h) {
     hg::StageArgs a{};
     a.K = h->K;
@@ -98,6 +117,7 @@ hg::StageArgs base_args(hg_handle *h) {
     a.dtr_out = h->dtr[h->ip_fused ? h->cur : 0];
     a.metric = h->metric;
     a.metric_kind = h->metric_kind;
+    a.affine = h->affine;
     a.face = h->face;
     a.forder = h->forder;
     a.egeo = h->egeo;
@@ -733,12 +753,21 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
                 }
             }
     }
-    std::vector<double> hat(PP), Dm(PP), lb(2 * P), lbw(2 * P), dlbw(2 * P), wv(P);
+    // lb, behind it lb hatD, lb D (per side) and lb lbw (side by side) of the kernels for parallelograms
+    std::vector<double> hat(PP), Dm(PP), lb(6 * P + 4, 0.0), lbw(2 * P), dlbw(2 * P), wv(P);
     for (int i = 0; i < P; ++i) {
         for (int l = 0; l < P; ++l) { hat[i * P + l] = sp.hatD[i][l]; Dm[i * P + l] = sp.D[i][l]; }
         for (int s = 0; s < 2; ++s) { lb[s * P + i] = sp.lb[s][i]; lbw[s * P + i] = sp.lbw[s][i]; dlbw[s * P + i] = sp.dlbw[s][i]; }
         wv[i] = sp.w[i];
     }
+    for (int s = 0; s < 2; ++s)
+        for (int i = 0; i < P; ++i) {
+            for (int l = 0; l < P; ++l) {
+                lb[(2 + s) * P + l] += sp.lb[s][i] * sp.hatD[i][l];
+                lb[(4 + s) * P + l] += sp.lb[s][i] * sp.D[i][l];
+            }
+            for (int o = 0; o < 2; ++o) lb[6 * P + 2 * s + o] += sp.lb[s][i] * sp.lbw[o][i];
+        }
     // ---- device allocations
     HG_CHECK(h->alloc(&h->Q, h->ndof));
     HG_CHECK(h->alloc(&h->G, h->ndof));
@@ -784,6 +813,27 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
         }
     } else if (line_metric(metric, K, P, metric_e)) {
         h->metric_kind = hg::METRIC_LINE;
+        // the kernels for parallelograms take a face's normal for all of its nodes and every lift from
+        // its own face node
+        bool plain = true;
+        for (const int4 &f : face) plain = plain && !(f.x & hg::FF_CURVED);
+        for (const int o : forder) plain = plain && !(o >> 8);
+        std::vector<double> reach(K, 0.0);
+        for (int e = 0; e < K; ++e)
+            for (const int v : m.el[els[e]].nodes)
+                for (int d = 0; d < 2; ++d) reach[e] = std::fmax(reach[e], std::fabs(m.pts[2 * v + d]));
+        h->affine = ph.ns && plain && parallelograms(metric_e, reach, K, P);
+        if (h->affine)   // behind the lines: 1/jac per element, from its sides (exact differences)
+            for (int e = 0; e < K; ++e) {
+                const hg::Elem &el = m.el[els[e]];
+                double d[2][2];   // along xi and eta: the mean of the two sides
+                for (int c = 0; c < 2; ++c) {
+                    auto x = [&](int v) { return m.pts[2 * el.nodes[v] + c]; };
+                    d[0][c] = 0.5 * ((x(1) - x(0)) + (x(2) - x(3)));
+                    d[1][c] = 0.5 * ((x(3) - x(0)) + (x(2) - x(1)));
+                }
+                metric_e.push_back(1.0 / (d[0][0] * d[1][1] - d[0][1] * d[1][0]));
+            }
     }
     HG_CHECK(upload_real(h, &h->metric, h->metric_kind == hg::METRIC_NODE ? metric : metric_e, h->mixed));
     if (!fmet.empty()) HG_CHECK(upload_real(h, &h->fmet, fmet, h->mixed));

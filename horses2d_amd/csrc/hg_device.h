@@ -74,7 +74,8 @@ struct StageArgs {
     void *dtr_out;
     const void *metric;         // 5 planes: Ja11, Ja12, Ja21, Ja22, 1/jac, per node or per element,
     int metric_kind;            // METRIC_NODE or METRIC_ELEM; METRIC_LINE: (Ja11, Ja21) at [e*P + i],
-                                // then (Ja12, Ja22) at [e*P + j]
+                                // then (Ja12, Ja22) at [e*P + j] (affine: then 1/jac per element)
+    int affine;                 // FP64 Navier-Stokes: METRIC_LINE, and every element a parallelogram
     const int4 *face;           // per element face record
     const int *forder;          // per element: faces sorted by global edge id (2 bits each)
     const double *egeo;         // edge geometry triplets (nx, ny, dS)

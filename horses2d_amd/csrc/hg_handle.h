@@ -44,6 +44,7 @@ struct hg_handle {
     bool vtr_valid = false;
     void *metric = nullptr, *fmet = nullptr;
     int metric_kind = hg::METRIC_NODE;
+    bool affine = false;    // StageArgs::affine
     int4 *face = nullptr;
     int *forder = nullptr;
     double *egeo = nullptr, *einvh = nullptr, *zone = nullptr;

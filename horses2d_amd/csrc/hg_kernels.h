@@ -161,6 +161,46 @@ __device__ __forceinline__ void face_trace(const T *X, int x0, const A *sLb, int
     }
 }
 
+// The same together with the derivative along the line at its end, sum of q(l) lbd(l) (lbd: lb D or lb
+// hatD, one row per side), from the same reads.
+template <int P, int NL, int UNROLL = P>
+__device__ __forceinline__ void face_trace_slope(const double *X, int x0, const double *sLb, const double *sLbd, int f,
+                                                 int k, double *out, double *nd) {
+    const int side = (f == 0 || f == 3) ? 0 : P;
+    constexpr int RS = Layout<P>::RS;
+    const bool horiz = (f == 0 || f == 2);
+    const int base = x0 + (horiz ? k : RS * k), step = horiz ? RS : 1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) out[c] = nd[c] = 0.0;
+#pragma unroll UNROLL
+    for (int l = 0; l < P; ++l) {
+        double v[4];
+        Quads<double, NL>::get(X, base + step * l, v);
+        const double b = sLb[side + l], d = sLbd[side + l];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            out[c] = fma(v[c], b, out[c]);
+            nd[c] = fma(v[c], d, nd[c]);
+        }
+    }
+}
+
+// Derivative along a face at its node k from the face's Q traces (an array of NF entries, f0 the face's
+// first), M the transposed D or hatD.
+template <int P, int NF, int UNROLL = P>
+__device__ __forceinline__ void face_tangent(const double *T, int f0, const double *M, int k, double *td) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) td[c] = 0.0;
+#pragma unroll UNROLL
+    for (int l = 0; l < P; ++l) {
+        double v[4];
+        Quads<double, NF>::get(T, f0 + l, v);
+        const double d = M[l * P + k];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) td[c] = fma(v[c], d, td[c]);
+    }
+}
+
 // The same for an eight-value array (two Quads arrays one after the other): one pass over the nodes.
 template <int P, int NL, int UNROLL = P, typename T, typename A>
 __device__ __forceinline__ void face_trace8(const T *X, int x0, const A *sLb, int f, int k, A *out) {
@@ -258,12 +298,32 @@ __device__ __forceinline__ const double *zone_state(const StageArgs &a, int flag
 }
 
 // BR1 solution flux at a face node: uStar n dS in both directions (DGViscous_BR1.f90:313-328;
-// boundary faces use the ghost state's uSB, DGViscousMethods.f90:786-917), stored as
-// out[0..3] = uStar dS and out[4..5] = (nx, ny); the lift forms (uStar dS) nx and (uStar dS) ny.
-// zd: the boundary's zone state (zone_state).
-template <typename R, bool XB>
+// boundary faces use the ghost state's uSB, DGViscousMethods.f90:786-917).  FP64: six values per face
+// node, uStar dS and (nx, ny), which the lift multiplies by lw n; FP32, whose sums keep the order (uStar
+// dS) nx lw: (uStar dS) nx and (uStar dS) ny, formed once here, as two Quads arrays.
+// zd: the boundary's zone state (zone_state); NF: face nodes of the tile, t: this one.
+template <typename R>
+constexpr int br1_width() { return sizeof(R) == 8 ? 6 : 8; }
+
+template <int NF, typename R>
+__device__ __forceinline__ void put_br1_flux(R *Fu, int t, const R *f, R nx, R ny) {
+    if constexpr (sizeof(R) == 8) {
+        R *out = Fu + t * 6;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) out[c] = f[c];
+        out[4] = nx; out[5] = ny;
+    } else {
+        R fx[4], fy[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) { fx[c] = f[c] * nx; fy[c] = f[c] * ny; }
+        Quads<R, NF>::put(Fu, t, fx);
+        Quads<R, NF>::put(Fu + 4 * NF, t, fy);
+    }
+}
+
+template <int NF, typename R, bool XB>
 __device__ __forceinline__ void br1_face_flux(const StageArgs &a, const Phys<R> &ph, int flags, const double *zd,
-                                              const R *qs, const R *qo, R nx, R ny, R dS, R *out) {
+                                              const R *qs, const R *qo, R nx, R ny, R dS, R *Fu, int t) {
     const int kind = flags & 15;
     R us[4];
     if (kind <= FK_PERIODIC) {
@@ -277,9 +337,7 @@ __device__ __forceinline__ void br1_face_flux(const StageArgs &a, const Phys<R> 
         // projected and signed by the mortar kernel (load_face put it in qo)
         if (flags & FF_MCURVED) {
             // a curved mortar edge: qo holds uStar dS nx already; the y terms follow separately
-#pragma unroll
-            for (int c = 0; c < 4; ++c) out[c] = qo[c];
-            out[4] = R(1); out[5] = R(0);
+            put_br1_flux<NF>(Fu, t, qo, R(1), R(0));
             return;
         }
 #pragma unroll
@@ -290,71 +348,108 @@ __device__ __forceinline__ void br1_face_flux(const StageArgs &a, const Phys<R> 
         ghost_state<R, XB>(kind, flags, zd, a.ph, ph, qs, nx, ny, uB, us, neu);
     }
 #pragma unroll
-    for (int c = 0; c < 4; ++c) out[c] = us[c] * dS;
-    out[4] = nx; out[5] = ny;
+    for (int c = 0; c < 4; ++c) us[c] = us[c] * dS;
+    put_br1_flux<NF>(Fu, t, us, nx, ny);
 }
 
 // BR1 gradient at node (i, j): ( -Vector_StdVolumeGreen(Q) + sum_faces Vector_StdFace(uStar) ) / jac
 // (DGViscous_BR1.f90:48-111, DGWeakIntegrals.f90:503-622), faces lifted in edge-id order.
 // q: the tile's state in the compute type (Quads; energy slot shifted in the FP32 form), Ja: its
-// metric (Quads: Ja11, Ja21, Ja12, Ja22), x0 the element's first entry in both, Fu: element uStar
-// fluxes [(f*P + k)*6] (see br1_face_flux), sHat: hatD transposed (hatD(i, l) at [l*P + i]).
+// metric (Quads: Ja11, Ja21, Ja12, Ja22), x0 the element's first entry in both, Fu: the tile's uStar
+// fluxes (see br1_face_flux), f0 the element's first face node, sHat: hatD transposed (hatD(i, l) at [l*P + i]).
 // Faces whose bit 8 + f is set in ord are curved p-non-conforming or subdivided edges, whose
 // lift terms come per direction from the mortar kernel (uStar dS n projected direction by
 // direction): the face lane stores the x terms with the "normal" (1, 0), and mortar_y_lift adds
 // the y terms afterwards.
-template <int P, int NL, typename R, int UNROLL = P>
-__device__ __forceinline__ void br1_node_gradient(const R *q, const R *Ja, int x0, const R *sHat, const R *Fu,
-                                                  const R *sLbw, int ord, int i, int j, R ijac, R *dq) {
-    // Every accumulator receives its xi terms (l = 0..P-1) then its eta terms; each state value
-    // is read once and used for both directions, and the metric-weighted derivative entry
-    // Ja * hatD is formed once per node for all four variables.
-    constexpr int RS = Layout<P>::RS;
-    using V = Quads<R, NL>;
-    R acc[8];
+template <int P, int NL, int NF, typename R, int UNROLL = P>
+__device__ __forceinline__ void br1_node_gradient(const R *q, const R *Ja, int x0, const R *sHat, const R *Fu, int f0,
+                                                  const R *sLbw, int ord, int i, int j, R ijac, R *dq,
+                                                  bool affine = false, R j11 = R(0), R j12 = R(0), R j21 = R(0),
+                                                  R j22 = R(0)) {
+    bool done = false;
+    if constexpr (sizeof(R) == 8) {
+        if (affine) {   // the metric out of the sums
+            R dxi[4] = {0, 0, 0, 0}, deta[4] = {0, 0, 0, 0};
+            // half unrolled up to P = 9, where the full loop spills a few registers
+#pragma unroll (UNROLL > 2 && P <= 9 ? (P + 1) / 2 : UNROLL)
+            for (int l = 0; l < P; ++l) {
+                const R hi = sHat[l * P + i], hj = sHat[l * P + j];
+                R vx[4], vy[4];
+                Quads<R, NL>::get(q, x0 + l + Layout<P>::RS * j, vx);
+                Quads<R, NL>::get(q, x0 + i + Layout<P>::RS * l, vy);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) acc[c] = R(0);
-#pragma unroll UNROLL
-    for (int l = 0; l < P; ++l) {
-        const int m = x0 + l + RS * j;
-        const R h = sHat[l * P + i];
-        R j11, j21, v[4];
-        V::get_half(Ja, m, 0, j11, j21);
-        V::get(q, m, v);
-        const R w0 = j11 * h, w2 = j21 * h;
+                for (int c = 0; c < 4; ++c) { dxi[c] += vx[c] * hi; deta[c] += vy[c] * hj; }
+            }
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            acc[c] += v[c] * w0;
-            acc[4 + c] += v[c] * w2;
+            for (int c = 0; c < 4; ++c) {
+                dq[c] = -(dxi[c] * j11 + deta[c] * j12);
+                dq[4 + c] = -(dxi[c] * j21 + deta[c] * j22);
+            }
+            done = true;
         }
     }
+    if (!done) {
+        // Every accumulator receives its xi terms (l = 0..P-1) then its eta terms; each state value
+        // is read once and used for both directions, and the metric-weighted derivative entry
+        // Ja * hatD is formed once per node for all four variables.
+        constexpr int RS = Layout<P>::RS;
+        using V = Quads<R, NL>;
+        R acc[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[c] = R(0);
 #pragma unroll UNROLL
-    for (int l = 0; l < P; ++l) {
-        const int m = x0 + i + RS * l;
-        const R h = sHat[l * P + j];
-        R j12, j22, v[4];
-        V::get_half(Ja, m, 1, j12, j22);
-        V::get(q, m, v);
-        const R w1 = j12 * h, w3 = j22 * h;
+        for (int l = 0; l < P; ++l) {
+            const int m = x0 + l + RS * j;
+            const R h = sHat[l * P + i];
+            R j11, j21, v[4];
+            V::get_half(Ja, m, 0, j11, j21);
+            V::get(q, m, v);
+            const R w0 = j11 * h, w2 = j21 * h;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            acc[c] += v[c] * w1;
-            acc[4 + c] += v[c] * w3;
+            for (int c = 0; c < 4; ++c) {
+                acc[c] += v[c] * w0;
+                acc[4 + c] += v[c] * w2;
+            }
         }
-    }
+#pragma unroll UNROLL
+        for (int l = 0; l < P; ++l) {
+            const int m = x0 + i + RS * l;
+            const R h = sHat[l * P + j];
+            R j12, j22, v[4];
+            V::get_half(Ja, m, 1, j12, j22);
+            V::get(q, m, v);
+            const R w1 = j12 * h, w3 = j22 * h;
 #pragma unroll
-    for (int c = 0; c < 8; ++c) dq[c] = -acc[c];
+            for (int c = 0; c < 4; ++c) {
+                acc[c] += v[c] * w1;
+                acc[4 + c] += v[c] * w3;
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) dq[c] = -acc[c];
+    }
 #pragma unroll
     for (int o = 0; o < 4; ++o) {
         const int f = (ord >> (2 * o)) & 3;
-        const R *F = Fu + (f * P + ((f == 0 || f == 2) ? i : j)) * 6;
+        const int xf = f0 + f * P + ((f == 0 || f == 2) ? i : j);
         const R lw = (f == 0) ? sLbw[j] : (f == 1) ? sLbw[P + i] : (f == 2) ? sLbw[P + j] : sLbw[i];
-        const R fnx = F[4], fny = F[5];
+        if constexpr (sizeof(R) == 8) {
+            const R *F = Fu + xf * 6;
+            const R wx = F[4] * lw, wy = F[5] * lw;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const R ux = F[c] * fnx, uy = F[c] * fny;
-            dq[c] += ux * lw;
-            dq[4 + c] += uy * lw;
+            for (int c = 0; c < 4; ++c) {
+                dq[c] += F[c] * wx;
+                dq[4 + c] += F[c] * wy;
+            }
+        } else {
+            R ux[4], uy[4];
+            Quads<R, NF>::get(Fu, xf, ux);
+            Quads<R, NF>::get(Fu + 4 * NF, xf, uy);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                dq[c] += ux[c] * lw;
+                dq[4 + c] += uy[c] * lw;
+            }
         }
     }
 #pragma unroll
@@ -404,12 +499,13 @@ __device__ __forceinline__ void ip_node_gradient(const R *q, int x0, const R *sD
     }
 }
 
-// Metric of node g, node n (= i + P j) of element e.  METRIC_NODE: five planes of nodes;
-// METRIC_ELEM: five planes of elements (FP32 form, element-constant metric); METRIC_LINE (FP64 form,
-// straight-sided elements): the derivatives of the bilinear map along eta depend on i alone and those
-// along xi on j alone, so two values per line of nodes replace 40 B per node, and the Jacobian and
-// its reciprocal are formed here in the host's operations, hence the same bits.  128 x 128 elements
-// at N = 6: the Euler stage 37.7 -> 33.2 us, the BR1 gradient kernel 27.0 -> 23.5 us.
+// Metric of node g, node n (= i + P j) of element e.  METRIC_NODE: five planes of nodes; METRIC_ELEM
+// (FP32 form): five planes of elements.  METRIC_LINE (FP64 form, straight-sided elements): the
+// derivatives of the bilinear map along eta depend on i alone and those along xi on j alone, so two
+// values per line of nodes replace 40 B per node, and the Jacobian and its reciprocal are formed here in
+// the host's operations, hence the same bits.  128 x 128 elements at N = 6: the Euler stage
+// 37.7 -> 33.2 us, the BR1 gradient kernel 27.0 -> 23.5 us.  Parallelograms: one reciprocal per element
+// behind the lines (128 x 128, N = 6, Navier-Stokes: 178.6 -> 176.5 us a step without the divisions).
 template <int P, typename R>
 __device__ __forceinline__ void load_metric(const StageArgs &a, int e, int n, int64_t g, R &j11, R &j12, R &j21, R &j22,
                                             R &ijac) {
@@ -418,6 +514,10 @@ __device__ __forceinline__ void load_metric(const StageArgs &a, int e, int n, in
             const double2 *L = (const double2 *)a.metric;
             const double2 e11 = L[(int64_t)e * P + n % P], e12 = L[(int64_t)(a.K + e) * P + n / P];
             j11 = e11.x; j21 = e11.y; j12 = e12.x; j22 = e12.y;
+            if (a.affine) {
+                ijac = ((const double *)a.metric)[4 * (int64_t)a.K * P + e];
+                return;
+            }
             double jac;
             {
 #pragma clang fp contract(off)
@@ -489,29 +589,47 @@ __device__ __forceinline__ void stored_trace(const StageArgs &a, int fe, int ff,
     for (int c = 0; c < 4; ++c) qs[c] = (R)o[c];
 }
 
-// This side's viscous flux at a face node from its Q trace qs and the element's nodal gradient
-// tile (two Quads arrays, x0 the element's first entry), times mu, stored in the VT layout (ViscousFluxes.f90:39-80, adiabatic
-// walls :279-318).  The gradient trace is accumulated in FP64 in the FP64 form and in FP32 in
-// the FP32 form (lbR: lb in the compute type).
+// mu times this side's viscous flux at a face node from its Q trace and gradient trace, in the VT layout
+// (ViscousFluxes.f90:39-80, adiabatic walls :279-318).
 // mdq: where a p-non-conforming face keeps its gradient trace for the mortar kernel (or null).
+template <typename R, typename TR>
+__device__ __forceinline__ void put_viscous_trace(const Phys<R> &ph, int flags, const R *qs, const R *ds, TR *o, R muf,
+                                                  double *mdq) {
+    if (mdq) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) mdq[c] = (double)ds[c];
+    }
+    R fv[4], gv[4];
+    if (is_adiabatic(flags)) adiabatic_flux(ph, qs, ds, fv, gv);
+    else viscous_flux(ph, qs, ds, fv, gv);
+    o[0] = (TR)(muf * fv[1]); o[1] = (TR)(muf * fv[2]); o[2] = (TR)(muf * fv[3]);
+    o[3] = (TR)(muf * gv[2]); o[4] = (TR)(muf * gv[3]); o[5] = TR(0);
+}
+
+// This side's viscous flux at a face node from its Q trace qs and the element's nodal gradient
+// tile (two Quads arrays, x0 the element's first entry).  The gradient trace is accumulated in FP64 in
+// the FP64 form and in FP32 in the FP32 form (lbR: lb in the compute type).
 template <int P, int NL, typename R, typename TR, int UNROLL = P>
 __device__ __forceinline__ void viscous_face_trace(const StageArgs &a, const Phys<R> &ph, int flags, const R *qs,
                                                    const R *sDQ, int x0, const double *sLb, const R *lbR, int ff,
                                                    int fk, TR *o, R muf, double *mdq = nullptr) {
-    R ds[8], fv[4], gv[4];
+    R ds[8];
     if constexpr (sizeof(R) == 4) {
         face_trace8<P, NL, UNROLL>(sDQ, x0, lbR, ff, fk, ds);
     } else {
         face_trace8<P, NL, UNROLL>(sDQ, x0, sLb, ff, fk, ds);
     }
-    if (mdq) {
+    put_viscous_trace<R, TR>(ph, flags, qs, ds, o, muf, mdq);
+}
+
+// Jacobian times the physical gradient, constant metric.
+__device__ __forceinline__ void affine_gradient(const double *dxi, const double *deta, double j11, double j12, double j21,
+                                                double j22, double *ds) {
 #pragma unroll
-        for (int c = 0; c < 8; ++c) mdq[c] = (double)ds[c];
+    for (int c = 0; c < 4; ++c) {
+        ds[c] = dxi[c] * j11 + deta[c] * j12;
+        ds[4 + c] = dxi[c] * j21 + deta[c] * j22;
     }
-    if (is_adiabatic(flags)) adiabatic_flux(ph, qs, ds, fv, gv);
-    else viscous_flux(ph, qs, ds, fv, gv);
-    o[0] = (TR)(muf * fv[1]); o[1] = (TR)(muf * fv[2]); o[2] = (TR)(muf * fv[3]);
-    o[3] = (TR)(muf * gv[2]); o[4] = (TR)(muf * gv[3]); o[5] = TR(0);
 }
 
 // ------------------------------------------------------------------ gradient trace kernel
@@ -525,7 +643,8 @@ struct GradSmem {
     struct Inputs {
         alignas(16) double sQ[sizeof(R) == 4 ? 2 : T::NL * 4];   // FP64 form: the state
         alignas(16) R sQf[sizeof(R) == 4 ? T::NL * 4 : 1];        // FP32 form: the compute-type state
-        alignas(16) R sJa[BR1 ? T::NL * 4 : 1];
+        // the metric; parallelograms, FP64: the faces' Q traces
+        alignas(16) R sJa[sizeof(R) == 8 ? (T::NL > T::NF ? T::NL : T::NF) * 4 : BR1 ? T::NL * 4 : 1];
     };
     // the state and the metric are dead once every node's gradient is formed: the gradient
     // tile takes their place
@@ -534,11 +653,121 @@ struct GradSmem {
         alignas(16) R sDQ[T::NL * 8];
     } u;
     alignas(16) double sLb[2 * P];
-    alignas(16) R sFu[BR1 ? T::NF * 6 : 1];
+    alignas(16) R sFu[BR1 ? T::NF * br1_width<R>() : 1];
     alignas(16) R sHat[BR1 ? T::PP : 1];
     alignas(16) R sLbw[4 * P];   // lbw, then lb in the compute type
     alignas(16) R sD[BR1 ? 1 : T::PP];
+    // parallelograms, FP64: lb M per side (M: hatD or D) and lb lbw of the sides; the face
+    // fluxes at the ends of their faces, [(s*4 + f)*2 + end]
+    alignas(16) R sLbd[sizeof(R) == 8 ? 2 * P + 4 : 1];
+    alignas(16) R sEnd[BR1 && sizeof(R) == 8 ? EPB * 8 * 4 : 1];
 };
+
+// gradient_body for parallelograms in FP64, whose metric is constant to rounding.  The physical gradient is then a constant
+// combination of the reference derivatives, and so its trace of theirs: along the face from the Q trace,
+// across it from the nodes of one line, each P terms.  A BR1 lift enters as the own and the opposite
+// face's value at this node and the two adjacent faces' values at this face's corners.  8 P fused
+// multiply-adds per variable and face node in place of 2 P (BR1: 4 P) per node and then 2 P per face node.
+// Bounded by latency and memory, no longer by LDS: 128 x 128, N = 6 24.6 -> 22.7 us, 61 x 53, N = 10
+// 16.6 -> 12.9 us.
+template <int P, int EPB, bool BR1, bool XB>
+__device__ __forceinline__ void gradient_affine(const StageArgs &a, const int e0, GradSmem<P, EPB, BR1, double> &S) {
+    using T = Tile<P, EPB>;
+    constexpr int NL = T::NL, NF = T::NF, NE = 8 * EPB;
+    using FaceV = Quads<double, NF>;
+    const int t = threadIdx.x, TPB = blockDim.x;
+    const Phys<double> ph(a.ph);
+    double *sQ = S.u.in.sQ, *sT = S.u.in.sJa, *sFu = S.sFu, *sM = BR1 ? S.sHat : S.sD;
+    if (t < 2 * P) {
+        S.sLb[t] = a.lb[t];
+        S.sLbd[t] = a.lb[(BR1 ? 2 : 4) * P + t];
+        if (BR1) S.sLbw[t] = a.lbw[t];
+    }
+    if (BR1 && t < 4) S.sLbd[2 * P + t] = a.lb[6 * P + t];
+    for (int x = t; x < T::PP; x += TPB) sM[x] = (BR1 ? a.hatD : a.D)[(x % P) * P + x / P];
+    const int s = t / T::PP, n = t % T::PP;
+    if (t < T::NN && e0 + s < a.K) {
+        double qg[4];
+        load_node(a.Q, (int64_t)e0 * T::PP + t, qg);
+        Quads<double, NL>::put(sQ, Layout<P>::at(s, n), qg);
+    }
+    const int fs = t / (4 * P), ff = (t / P) % 4, fk = t % P, fe = e0 + fs;
+    const bool face_active = t < NF && fe < a.K;
+    int4 fr = make_int4(0, 0, 0, 0);
+    double qs[4] = {0.0, 0.0, 0.0, 0.0}, j11 = 0.0, j12 = 0.0, j21 = 0.0, j22 = 0.0, ijac = 1.0;
+    if (face_active) {
+        stored_trace<P, double, double>(a, fe, ff, fk, qs);
+        const int fi = (ff & 1) ? (ff == 1 ? P - 1 : 0) : fk, fj = (ff & 1) ? fk : (ff == 2 ? P - 1 : 0);
+        load_metric<P, double>(a, fe, fi + P * fj, 0, j11, j12, j21, j22, ijac);   // of the nearest node
+        FaceV::put(sT, t, qs);
+        if constexpr (BR1) {
+            double nx, ny, dS, qo[4] = {0.0, 0.0, 0.0, 0.0};
+            int64_t nslot;
+            load_face<P, double, double>(a, fe, ff, fk, fr, nx, ny, dS, qo, nslot);
+            br1_face_flux<NF, double, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs,
+                                          qo, nx, ny, dS, sFu, t);
+        } else {
+            fr = a.face[fe * 4 + ff];
+        }
+    }
+    __syncthreads();
+    double ds[8];
+    if (face_active) {
+        const bool horiz = ff == 0 || ff == 2;
+        double qt[4], nd[4], td[4];
+        face_trace_slope<P, NL>(sQ, fs * Layout<P>::ES, S.sLb, S.sLbd, ff, fk, qt, nd);
+        face_tangent<P, NF>(sT, (fs * 4 + ff) * P, sM, fk, td);
+        affine_gradient(horiz ? td : nd, horiz ? nd : td, j11, j12, j21, j22, ds);
+    }
+    if constexpr (BR1) {
+        // by lanes that have no face node, where the tile has enough
+        constexpr int NF64 = (NF + 63) / 64 * 64, OFF = NF64 + NE <= T::TPB ? NF64 : NF + NE <= T::TPB ? NF : 0;
+        const int x = t - OFF;
+        if (x >= 0 && x < NE && e0 + x / 8 < a.K) {
+            const double *lb = S.sLb + (x & 1) * P, *F = sFu + (x >> 1) * P * 6;
+            double v[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+            for (int l = 0; l < P; ++l)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) v[c] = fma(F[l * 6 + c], lb[l], v[c]);
+            Quads<double, NE>::put(S.sEnd, x, v);
+        }
+        __syncthreads();
+        if (face_active) {
+#pragma unroll
+            for (int c = 0; c < 8; ++c) ds[c] = -ds[c];
+            const int side = (ff == 0 || ff == 3) ? 0 : 1;
+#pragma unroll
+            for (int o = 0; o < 4; ++o) {
+                // the own face, the opposite one, the adjacent ones at their sides 0 and 1
+                const int gf = o < 2 ? (ff ^ (2 * o)) : (ff & 1) ? (o == 2 ? 0 : 2) : (o == 2 ? 3 : 1);
+                const double lw = o < 2 ? S.sLbd[2 * P + 2 * side + (side ^ o)] : S.sLbw[(o - 2) * P + fk];
+                const int xf = (fs * 4 + gf) * P;
+                double F[4];
+                if (o < 2) {
+#pragma unroll
+                    for (int c = 0; c < 4; ++c) F[c] = sFu[(xf + fk) * 6 + c];
+                } else {
+                    Quads<double, NE>::get(S.sEnd, (fs * 4 + gf) * 2 + side, F);
+                }
+                const double wx = sFu[xf * 6 + 4] * lw, wy = sFu[xf * 6 + 5] * lw;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    ds[c] += F[c] * wx;
+                    ds[4 + c] += F[c] * wy;
+                }
+            }
+        }
+    }
+    if (face_active) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) ds[c] *= ijac;
+        const double muf = XB ? face_mu<double>(a, ph, fe, fr) : ph.mu;
+        const int64_t slot = (int64_t)(fe * 4 + ff) * P + fk;
+        double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + slot * 8 : nullptr;
+        put_viscous_trace<double, double>(ph, fr.x, qs, ds, (double *)a.dtr_out + slot * VT, muf, mdq);
+    }
+}
 
 // One element tile [e0, e0+EPB) of the gradient; any workgroup size >= Tile<P, EPB>::TPB.
 // XB: the Euler-wall, Dirichlet and pressure boundary kinds are compiled in.
@@ -547,6 +776,12 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
     using T = Tile<P, EPB>;
     constexpr int PP = T::PP, NN = T::NN, NF = T::NF;
     const int TPB = blockDim.x;
+    if constexpr (sizeof(R) == 8) {
+        if (a.affine) {
+            gradient_affine<P, EPB, BR1, XB>(a, e0, S);
+            return;
+        }
+    }
     double *sQ = S.u.in.sQ, *sLb = S.sLb;
     R *sDQ = S.u.sDQ, *sJa = S.u.in.sJa, *sFu = S.sFu, *sHat = S.sHat, *sLbw = S.sLbw, *sD = S.sD;
     const int t = threadIdx.x;
@@ -591,14 +826,14 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
         stored_trace<P, R, TR>(a, fe, ff, fk, qs);
     }
     if (BR1 && face_active)
-        br1_face_flux<R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx, ny,
-                             dS, sFu + t * 6);
+        br1_face_flux<NF, R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx,
+                                 ny, dS, sFu, t);
     __syncthreads();
     R dq[8];
     if (node_active) {
         const int i = n % P, j = n / P;
         if (BR1) {
-            br1_node_gradient<P, NL, R>(sQr, sJa, x0, sHat, sFu + s * 4 * P * 6, sLbw, ord, i, j, ijac, dq);
+            br1_node_gradient<P, NL, NF, R>(sQr, sJa, x0, sHat, sFu, s * 4 * P, sLbw, ord, i, j, ijac, dq);
             if (ord >> 8) mortar_y_lift<P, R>(a.mustar + (int64_t)e * 4 * P * 8, sLbw, ord, i, j, ijac, dq);
         }
         else ip_node_gradient<P, NL, R>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dq);
@@ -641,7 +876,7 @@ struct StageSmem {
     // the face fluxes (BR1: uStar fluxes during the gradient phase); once every wavefront has
     // lifted them, the residual maxima
     union {
-        alignas(16) R sF[NS && !IP ? T::NF * 6 : T::NF * 4];
+        alignas(16) R sF[NS && !IP ? T::NF * br1_width<R>() : T::NF * 4];
         uint64_t sRes[4][4];
     };
     // IP gradient-face terms: the face phase's contravariant fluxes, then (same arrays) the
@@ -687,6 +922,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     const int t = threadIdx.x;
     const Phys<R> ph(a.ph);
     const bool ipgrad = IP && a.ph.ip_gradflux;
+    const bool affine = NS && sizeof(R) == 8 && a.affine;   // constant metric
     if (a.resid_max && !a.do_resid && e0 == 0 && t < 4) a.resid_max[t * kResidStride] = 0.0;
     if (t < 2 * P) {
         sLb[t] = a.lb[t]; sLbw[t] = (R)a.lbw[t]; sDlbw[t] = (R)a.dlbw[t];
@@ -723,7 +959,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         ord = a.forder[e];
         Quads<double, NL>::put(sQ, xn, qg);
         if constexpr (COPY) put_slots<NL, R>(a.ph, sCG, xn, qg);
-        if (BR1) {
+        if (BR1 && !affine) {
             const R jv[4] = {j11, j21, j12, j22};
             NodeV::put(sCF, xn, jv);
         }
@@ -740,8 +976,8 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         stored_trace<P, R, TR>(a, fe, ff, fk, qs);
     }
     if (BR1 && face_active)
-        br1_face_flux<R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx, ny,
-                             dS, sF + t * 6);
+        br1_face_flux<NF, R, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs, qo, nx,
+                                 ny, dS, sF, t);
     if (NS) __syncthreads();
 
     // ---- own nodal gradient (Navier-Stokes), kept in registers for the node phase
@@ -753,7 +989,8 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     if (NS && node_active) {
         const int i = n % P, j = n / P;
         if (BR1) {
-            br1_node_gradient<P, NL, R, UNROLL>(sQr, sCF, x0, sHat, sF + s * 4 * P * 6, sLbw, ord, i, j, ijac, dq);
+            br1_node_gradient<P, NL, NF, R, UNROLL>(sQr, sCF, x0, sHat, sF, s * 4 * P, sLbw, ord, i, j, ijac, dq, affine,
+                                                    j11, j12, j21, j22);
             if (ord >> 8) mortar_y_lift<P, R>(a.mustar + (int64_t)e * 4 * P * 8, sLbw, ord, i, j, ijac, dq);
         }
         else ip_node_gradient<P, NL, R, UNROLL>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dq);
@@ -1086,9 +1323,13 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     }
     if (a.mode == 0) {
         R qn[4];   // the next stage's own Q trace in the compute type (IP epilogue)
+        constexpr bool SLOPE = IP && sizeof(R) == 8;
+        double nd[4] = {0.0, 0.0, 0.0, 0.0};
         if (face_active) {
             double tq[4];
-            face_trace<P, NL, UNROLL>(sQ, fs * Layout<P>::ES, sLb, ff, fk, tq);
+            if (SLOPE && affine)
+                face_trace_slope<P, NL, UNROLL>(sQ, fs * Layout<P>::ES, sLb, a.lb + 4 * P, ff, fk, tq, nd);
+            else face_trace<P, NL, UNROLL>(sQ, fs * Layout<P>::ES, sLb, ff, fk, tq);
             tq[3] = slot_energy<TR>(a.ph, tq[3]);
             TR *o = (TR *)a.tr_out + ((int64_t)(fe * 4 + ff) * P + fk) * 4;
 #pragma unroll
@@ -1097,6 +1338,27 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             for (int c = 0; c < 4; ++c) qn[c] = (R)(TR)tq[c];
         }
         if constexpr (IP) {
+          if constexpr (SLOPE) {
+            if (affine && (!XB || a.ip_epi)) {
+                // the gradient's trace from the face's Q trace and the line across it, as gradient_affine
+                if (face_active) FaceV::put(sU, t, qn);
+                __syncthreads();
+                if (face_active) {
+                    const bool horiz = ff == 0 || ff == 2;
+                    double td[4], ds[8], m11, m12, m21, m22, mij;
+                    const int fi = horiz ? fk : (ff == 1 ? P - 1 : 0), fj = horiz ? (ff == 2 ? P - 1 : 0) : fk;
+                    load_metric<P, double>(a, fe, fi + P * fj, 0, m11, m12, m21, m22, mij);
+                    face_tangent<P, NF, UNROLL>(sU, (fs * 4 + ff) * P, sD, fk, td);
+                    affine_gradient(horiz ? td : nd, horiz ? nd : td, m11, m12, m21, m22, ds);
+#pragma unroll
+                    for (int c = 0; c < 8; ++c) ds[c] *= mij;
+                    const int64_t slot = (int64_t)(fe * 4 + ff) * P + fk;
+                    double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + slot * 8 : nullptr;
+                    put_viscous_trace<double, double>(ph, fr.x, qn, ds, (double *)a.dtr_out + slot * VT, ph.mu, mdq);
+                }
+                return;
+            }
+          }
           if (!XB || a.ip_epi) {   // uniform: the launch's flag
             // the updated state in the compute type (FP32: a fresh copy, the node phase
             // overwrote the first one), the broken gradient, its traces and this side's
