@@ -115,6 +115,7 @@ hg::StageArgs base_args(hg_handle *h) {
     a.QDot = h->QDot;
     a.dtr = h->dtr[h->ip_fused ? h->cur : 0];
     a.dtr_out = h->dtr[h->ip_fused ? h->cur : 0];
+    a.vt = h->vt;
     a.metric = h->metric;
     a.metric_kind = h->metric_kind;
     a.affine = h->affine;
@@ -641,6 +642,7 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
         egeo.push_back(ed.n[1]);
         egeo.push_back(0.5 * ed.dS[0]);
     }
+    h->vt = h->mixed ? hg::VT_FLUX : hg::VT_NORMAL;
     std::vector<int4> face(4 * (size_t)K);
     std::vector<int> forder(K);
     std::vector<double> zone(8 * std::max<size_t>(m.zones.size(), 1), 0.0);
@@ -685,6 +687,9 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
                     if (loc[pe.quads[0]] < 0)
                         return set_err("hg_create: periodic edges between elements of different orders");
                     y = loc[pe.quads[0]] * 4 + (pe.loc[0] - 1);
+                    // paired by one coordinate of their ends: parallel to rounding, or not
+                    if (!(std::fabs(ed.n[0] + pe.n[0]) <= 1e-13 && std::fabs(ed.n[1] + pe.n[1]) <= 1e-13))
+                        h->vt = hg::VT_FLUX;
                     if (ed.inverse) flags |= hg::FF_REV;
                 } else {
                     switch (Z.type) {
@@ -782,7 +787,7 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
         // (the Laplacian type leaves mu alone: its viscous traces do not wait for the indicator)
         h->ip_fused = ph.viscous == HG_VISCOUS_IP && (!ph.ad || h->lap);
         for (int b = 0; b < (h->ip_fused ? 2 : 1); ++b)
-            HG_CHECK(h->alloc_raw(&h->dtr[b], (size_t)K * 4 * P * hg::VT * rs));
+            HG_CHECK(h->alloc_raw(&h->dtr[b], (size_t)K * 4 * P * h->vt * rs));
     }
     // The FP32 form stores one metric record per element when every element's metric is
     // constant to FP32 resolution (straight-sided parallelograms): each node's value differs
@@ -1619,7 +1624,7 @@ int hg_surface_integrals(hg_handle *h, int32_t marker, double out[9]) {
         hg::mark_last_evaluation(h, h->cur);
     }
     if (n > 0)
-        HG_CHECK(hg::launch_surface_integrals(h->mixed, h->bslots + first, n, h->P, tr, vtr, h->face,
+        HG_CHECK(hg::launch_surface_integrals(h->mixed, h->bslots + first, n, h->P, tr, vtr, h->vt, h->face,
                                               h->egeo, h->w, h->ph.gm1, h->mixed ? h->ph.Eref : 0.0,
                                               (h->ph.ad && !h->lap) ? h->mu_a : nullptr, h->ph.mu, h->monitor_out,
                                               h->stream));

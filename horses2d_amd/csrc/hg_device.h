@@ -33,9 +33,14 @@ constexpr int FF_FSTATE = 1 << 13;   // boundary face whose zone state comes per
                                      // boundary-state function (StageArgs::fstate)
 constexpr int FF_MCURVED = 1 << 14;  // mortar face of a curved edge: BR1 uStar dS n per direction
 
-// Viscous face-flux traces: per element face node, mu times this side's viscous flux from its
-// own Q and gradient traces, (f1, f2, f3, g2, g3) and one pad (f0 = g0 = 0, g1 = f2).
-constexpr int VT = 6;
+// Values of a viscous face-flux trace, per element face node: mu times this side's viscous flux from its
+// own Q and gradient traces.  VT_FLUX: (f1, f2, f3, g2, g3) (f0 = g0 = 0, g1 = f2).  VT_NORMAL: its
+// components 1 to 3 along the edge's normal (a periodic face: its own outward normal), which is all
+// that the face flux and the surface stress need; the FP64 form, unless two periodic edges paired by
+// their end points are not parallel.  FP32 stays with VT_FLUX, whose averages are rounded per direction.
+// Memory-bound kernels read and write these: six values a node -> three, 128 x 128, N = 6, BR1 179.6 ->
+// 170.8 us a step; six -> five, FP32 form, 160 x 160 O-grid, N = 7 239 -> 234 us.
+constexpr int VT_FLUX = 5, VT_NORMAL = 3;
 
 // How a handle's metric is stored (load_metric): per node, per element (FP32 form, every element's
 // metric constant), per line of nodes (FP64 form, every element straight-sided).
@@ -70,8 +75,9 @@ struct StageArgs {
     double *QDot;               // derivative output (derivative-only mode) or nullptr
     const void *tr_in;          // Q traces [(e*4+f)*P + k][4] (FP64 or FP32)
     void *tr_out;               // next-stage Q traces
-    const void *dtr;            // viscous face-flux traces [(e*4+f)*P + k][VT] (FP64 or FP32)
+    const void *dtr;            // viscous face-flux traces [(e*4+f)*P + k][vt] (FP64 or FP32)
     void *dtr_out;
+    int vt;                     // VT_FLUX or VT_NORMAL (FP64)
     const void *metric;         // 5 planes: Ja11, Ja12, Ja21, Ja22, 1/jac, per node or per element,
     int metric_kind;            // METRIC_NODE or METRIC_ELEM; METRIC_LINE: (Ja11, Ja21) at [e*P + i],
                                 // then (Ja12, Ja22) at [e*P + j] (affine: then 1/jac per element)
@@ -242,7 +248,7 @@ hipError_t launch_volume_integrals(int P, const double *Q, const double *jac, co
 // Surface monitors of one zone (QuadMesh_Integrals.incf:67-346) over its boundary face slots
 // (element*4 + face): out[9] = Surface, pressure, density, pressure force (2), mass-flow, flow,
 // viscous force (2); vtr null for Euler.  Eref: the FP32 form's energy-slot shift.
-hipError_t launch_surface_integrals(bool mixed, const int *slots, int nslots, int P, const void *tr, const void *vtr,
+hipError_t launch_surface_integrals(bool mixed, const int *slots, int nslots, int P, const void *tr, const void *vtr, int vt,
                                     const int4 *face, const double *egeo, const double *w, double gm1, double Eref,
                                     const double *mu_a, double mu, double *out, hipStream_t s);
 // Jumps-based artificial viscosity per element from the stage's Q traces (and boundary states).

@@ -149,10 +149,10 @@ __global__ __launch_bounds__(1024) void k_cons_final(const double *partial, int 
 // strided share of the zone's face nodes from the stored element-side Q traces (the energy slot
 // shifted back by Eref in the FP32 form) and, for Navier-Stokes, the stored viscous face-flux
 // traces, whose momentum components are the stress tensor (mu (f1, f2, g2) = tau_xx, tau_xy,
-// tau_yy, ViscousFluxes.f90:416-461); then a fixed-order reduction.
+// tau_yy, ViscousFluxes.f90:416-461) or its product with the normal (VT_NORMAL); then a fixed-order reduction.
 template <typename TR>
 __global__ __launch_bounds__(1024) void k_surface_integrals(const int *slots, int nslots, int P, const TR *tr,
-                                                            const TR *vtr, const int4 *face, const double *egeo,
+                                                            const TR *vtr, int vt, const int4 *face, const double *egeo,
                                                             const double *w, double gm1, double Eref,
                                                             const double *mu_a, double mu, double *out) {
     __shared__ double s[16][9];
@@ -177,12 +177,17 @@ __global__ __launch_bounds__(1024) void k_surface_integrals(const int *slots, in
         acc[5] += wq * un * dS;
         acc[6] += wq * un * dS / r;
         if (vtr) {
-            const TR *v = vtr + ((int64_t)slot * P + k) * VT;
+            const TR *v = vtr + ((int64_t)slot * P + k) * vt;
             // the traces carry mu + mu_a of the (boundary) face; the monitor's stress has mu
             const double sc = mu_a ? mu / (mu + mu_a[slot >> 2]) : 1.0;
-            const double txx = v[0] * sc, txy = v[1] * sc, tyy = v[3] * sc;
-            acc[7] += wq * (txx * nx + txy * ny) * dS;
-            acc[8] += wq * (txy * nx + tyy * ny) * dS;
+            if (vt == VT_NORMAL) {
+                acc[7] += wq * (v[0] * sc) * dS;
+                acc[8] += wq * (v[1] * sc) * dS;
+            } else {
+                const double txx = v[0] * sc, txy = v[1] * sc, tyy = v[3] * sc;
+                acc[7] += wq * (txx * nx + txy * ny) * dS;
+                acc[8] += wq * (txy * nx + tyy * ny) * dS;
+            }
         }
     }
 #pragma unroll
@@ -439,15 +444,15 @@ hipError_t launch_volume_integrals(int P, const double *Q, const double *jac, co
     return hipGetLastError();
 }
 
-hipError_t launch_surface_integrals(bool mixed, const int *slots, int nslots, int P, const void *tr, const void *vtr,
+hipError_t launch_surface_integrals(bool mixed, const int *slots, int nslots, int P, const void *tr, const void *vtr, int vt,
                                     const int4 *face, const double *egeo, const double *w, double gm1, double Eref,
                                     const double *mu_a, double mu, double *out, hipStream_t st) {
     if (mixed)
         hipLaunchKernelGGL((k_surface_integrals<float>), dim3(1), dim3(1024), 0, st, slots, nslots, P,
-                           (const float *)tr, (const float *)vtr, face, egeo, w, gm1, Eref, mu_a, mu, out);
+                           (const float *)tr, (const float *)vtr, vt, face, egeo, w, gm1, Eref, mu_a, mu, out);
     else
         hipLaunchKernelGGL((k_surface_integrals<double>), dim3(1), dim3(1024), 0, st, slots, nslots, P,
-                           (const double *)tr, (const double *)vtr, face, egeo, w, gm1, Eref, mu_a, mu, out);
+                           (const double *)tr, (const double *)vtr, vt, face, egeo, w, gm1, Eref, mu_a, mu, out);
     return hipGetLastError();
 }
 

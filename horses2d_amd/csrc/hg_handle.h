@@ -45,6 +45,7 @@ struct hg_handle {
     void *metric = nullptr, *fmet = nullptr;
     int metric_kind = hg::METRIC_NODE;
     bool affine = false;    // StageArgs::affine
+    int vt = hg::VT_FLUX;   // values of a viscous flux trace
     int4 *face = nullptr;
     int *forder = nullptr;
     double *egeo = nullptr, *einvh = nullptr, *zone = nullptr;

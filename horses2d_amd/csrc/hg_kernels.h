@@ -3,9 +3,9 @@
 // Data layout in HBM (uniform polynomial order P = N+1 per handle):
 //   Q, G      : FP64, reference layout  Q[(e*P*P + i + P*j)*4 + eq]
 //   traces    : [(e*4 + f)*P + k][4]  element-local face orientation, FP64 or FP32
-//   viscous flux traces: [(e*4 + f)*P + k][VT], FP64 or FP32: mu times each side's viscous
-//               flux at its face nodes (the gradient itself is never stored: the nodal
-//               gradient is recomputed inside each stage)
+//   viscous flux traces: [(e*4 + f)*P + k][vt], FP64 or FP32: mu times each side's viscous
+//               flux at its face nodes, in FP64 its normal component (the gradient itself is never
+//               stored: the nodal gradient is recomputed inside each stage)
 //   metric    : five planes of e*P*P+n: Ja11, Ja12, Ja21, Ja22, 1/jac (FP64 or FP32; the FP32
 //               form stores one record per element when the metric is element-constant, the FP64
 //               form one per line of nodes when every element is straight-sided); the
@@ -573,7 +573,31 @@ __device__ __forceinline__ void load_face(const StageArgs &a, int fe, int ff, in
     }
 }
 
-// mu (f, g) of one side of a face node from its viscous flux trace (layout of VT).
+// Values of a stored viscous flux trace that a stage keeps.
+template <typename R>
+constexpr int vis_width() { return sizeof(R) == 8 ? VT_NORMAL : VT_FLUX; }
+
+// One side's viscous flux trace of a face node.  FP64: its components along (nx, ny); opposite: stored
+// along the opposite normal (the partner of a periodic face).
+template <typename R, typename TR>
+__device__ __forceinline__ void load_viscous_trace(const StageArgs &a, int64_t slot, R nx, R ny, bool opposite, R *v) {
+    if constexpr (sizeof(R) == 4) {
+        const TR *o = (const TR *)a.dtr + slot * VT_FLUX;
+#pragma unroll
+        for (int c = 0; c < VT_FLUX; ++c) v[c] = (R)o[c];
+    } else if (a.vt == VT_NORMAL) {
+        const TR *o = (const TR *)a.dtr + slot * VT_NORMAL;
+#pragma unroll
+        for (int c = 0; c < VT_NORMAL; ++c) v[c] = opposite ? -o[c] : o[c];
+    } else {
+        const TR *o = (const TR *)a.dtr + slot * VT_FLUX;
+        v[0] = o[0] * nx + o[1] * ny;
+        v[1] = o[1] * nx + o[3] * ny;
+        v[2] = o[2] * nx + o[4] * ny;
+    }
+}
+
+// mu (f, g) of one side of a face node from its viscous flux trace (FP32 form).
 template <typename R>
 __device__ __forceinline__ void viscous_trace_flux(const R *v, R *f, R *g) {
     f[0] = R(0); f[1] = v[0]; f[2] = v[1]; f[3] = v[2];
@@ -589,12 +613,12 @@ __device__ __forceinline__ void stored_trace(const StageArgs &a, int fe, int ff,
     for (int c = 0; c < 4; ++c) qs[c] = (R)o[c];
 }
 
-// mu times this side's viscous flux at a face node from its Q trace and gradient trace, in the VT layout
-// (ViscousFluxes.f90:39-80, adiabatic walls :279-318).
+// mu times this side's viscous flux at a face node from its Q trace and gradient trace
+// (ViscousFluxes.f90:39-80, adiabatic walls :279-318), stored at the face node's slot of the traces.
 // mdq: where a p-non-conforming face keeps its gradient trace for the mortar kernel (or null).
 template <typename R, typename TR>
-__device__ __forceinline__ void put_viscous_trace(const Phys<R> &ph, int flags, const R *qs, const R *ds, TR *o, R muf,
-                                                  double *mdq) {
+__device__ __forceinline__ void put_viscous_trace(const StageArgs &a, const Phys<R> &ph, int flags, const R *qs,
+                                                  const R *ds, int64_t slot, R nx, R ny, R muf, double *mdq) {
     if (mdq) {
 #pragma unroll
         for (int c = 0; c < 8; ++c) mdq[c] = (double)ds[c];
@@ -602,8 +626,15 @@ __device__ __forceinline__ void put_viscous_trace(const Phys<R> &ph, int flags, 
     R fv[4], gv[4];
     if (is_adiabatic(flags)) adiabatic_flux(ph, qs, ds, fv, gv);
     else viscous_flux(ph, qs, ds, fv, gv);
-    o[0] = (TR)(muf * fv[1]); o[1] = (TR)(muf * fv[2]); o[2] = (TR)(muf * fv[3]);
-    o[3] = (TR)(muf * gv[2]); o[4] = (TR)(muf * gv[3]); o[5] = TR(0);
+    if (sizeof(R) == 8 && a.vt == VT_NORMAL) {
+        TR *o = (TR *)a.dtr_out + slot * VT_NORMAL;
+#pragma unroll
+        for (int c = 0; c < VT_NORMAL; ++c) o[c] = (TR)(muf * (fv[c + 1] * nx + gv[c + 1] * ny));
+    } else {
+        TR *o = (TR *)a.dtr_out + slot * VT_FLUX;
+        o[0] = (TR)(muf * fv[1]); o[1] = (TR)(muf * fv[2]); o[2] = (TR)(muf * fv[3]);
+        o[3] = (TR)(muf * gv[2]); o[4] = (TR)(muf * gv[3]);
+    }
 }
 
 // This side's viscous flux at a face node from its Q trace qs and the element's nodal gradient
@@ -612,14 +643,14 @@ __device__ __forceinline__ void put_viscous_trace(const Phys<R> &ph, int flags, 
 template <int P, int NL, typename R, typename TR, int UNROLL = P>
 __device__ __forceinline__ void viscous_face_trace(const StageArgs &a, const Phys<R> &ph, int flags, const R *qs,
                                                    const R *sDQ, int x0, const double *sLb, const R *lbR, int ff,
-                                                   int fk, TR *o, R muf, double *mdq = nullptr) {
+                                                   int fk, int64_t slot, R nx, R ny, R muf, double *mdq) {
     R ds[8];
     if constexpr (sizeof(R) == 4) {
         face_trace8<P, NL, UNROLL>(sDQ, x0, lbR, ff, fk, ds);
     } else {
         face_trace8<P, NL, UNROLL>(sDQ, x0, sLb, ff, fk, ds);
     }
-    put_viscous_trace<R, TR>(ph, flags, qs, ds, o, muf, mdq);
+    put_viscous_trace<R, TR>(a, ph, flags, qs, ds, slot, nx, ny, muf, mdq);
 }
 
 // Jacobian times the physical gradient, constant metric.
@@ -694,21 +725,18 @@ __device__ __forceinline__ void gradient_affine(const StageArgs &a, const int e0
     const int fs = t / (4 * P), ff = (t / P) % 4, fk = t % P, fe = e0 + fs;
     const bool face_active = t < NF && fe < a.K;
     int4 fr = make_int4(0, 0, 0, 0);
-    double qs[4] = {0.0, 0.0, 0.0, 0.0}, j11 = 0.0, j12 = 0.0, j21 = 0.0, j22 = 0.0, ijac = 1.0;
+    double nx = 0.0, ny = 0.0, qs[4] = {0.0, 0.0, 0.0, 0.0}, j11 = 0.0, j12 = 0.0, j21 = 0.0, j22 = 0.0, ijac = 1.0;
     if (face_active) {
         stored_trace<P, double, double>(a, fe, ff, fk, qs);
         const int fi = (ff & 1) ? (ff == 1 ? P - 1 : 0) : fk, fj = (ff & 1) ? fk : (ff == 2 ? P - 1 : 0);
         load_metric<P, double>(a, fe, fi + P * fj, 0, j11, j12, j21, j22, ijac);   // of the nearest node
         FaceV::put(sT, t, qs);
-        if constexpr (BR1) {
-            double nx, ny, dS, qo[4] = {0.0, 0.0, 0.0, 0.0};
-            int64_t nslot;
-            load_face<P, double, double>(a, fe, ff, fk, fr, nx, ny, dS, qo, nslot);
+        double dS, qo[4] = {0.0, 0.0, 0.0, 0.0};
+        int64_t nslot;
+        load_face<P, double, double>(a, fe, ff, fk, fr, nx, ny, dS, qo, nslot);
+        if constexpr (BR1)
             br1_face_flux<NF, double, XB>(a, ph, fr.x, zone_state(a, fr.x, fr.y, (int64_t)(fe * 4 + ff) * P + fk), qs,
                                           qo, nx, ny, dS, sFu, t);
-        } else {
-            fr = a.face[fe * 4 + ff];
-        }
     }
     __syncthreads();
     double ds[8];
@@ -765,7 +793,7 @@ __device__ __forceinline__ void gradient_affine(const StageArgs &a, const int e0
         const double muf = XB ? face_mu<double>(a, ph, fe, fr) : ph.mu;
         const int64_t slot = (int64_t)(fe * 4 + ff) * P + fk;
         double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + slot * 8 : nullptr;
-        put_viscous_trace<double, double>(ph, fr.x, qs, ds, (double *)a.dtr_out + slot * VT, muf, mdq);
+        put_viscous_trace<double, double>(a, ph, fr.x, qs, ds, slot, nx, ny, muf, mdq);
     }
 }
 
@@ -821,8 +849,7 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
     int64_t nslot = 0;
     R qs[4] = {R(0), R(0), R(0), R(0)};
     if (face_active) {
-        if (BR1) load_face<P, R, TR>(a, fe, ff, fk, fr, nx, ny, dS, qo, nslot);
-        else fr = a.face[fe * 4 + ff];
+        load_face<P, R, TR>(a, fe, ff, fk, fr, nx, ny, dS, qo, nslot);
         stored_trace<P, R, TR>(a, fe, ff, fk, qs);
     }
     if (BR1 && face_active)
@@ -846,9 +873,10 @@ __device__ __forceinline__ void gradient_body(const StageArgs &a, const int e0, 
     __syncthreads();
     if (face_active) {
         const R muf = XB ? face_mu<R>(a, ph, fe, fr) : ph.mu;
-        double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + ((int64_t)(fe * 4 + ff) * P + fk) * 8 : nullptr;
-        viscous_face_trace<P, NL, R, TR>(a, ph, fr.x, qs, sDQ, fs * Layout<P>::ES, sLb, sLbw + 2 * P, ff, fk,
-                                         (TR *)a.dtr_out + ((int64_t)(fe * 4 + ff) * P + fk) * VT, muf, mdq);
+        const int64_t slot = (int64_t)(fe * 4 + ff) * P + fk;
+        double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + slot * 8 : nullptr;
+        viscous_face_trace<P, NL, R, TR>(a, ph, fr.x, qs, sDQ, fs * Layout<P>::ES, sLb, sLbw + 2 * P, ff, fk, slot, nx,
+                                         ny, muf, mdq);
     }
 }
 
@@ -997,19 +1025,19 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
         if (LAPG && a.lap) ip_node_gradient<P, NL, R, UNROLL>(sQr, x0, sD, i, j, j11, j12, j21, j22, ijac, dqi);
     }
     // the neighbour's viscous flux trace, issued before the barrier and consumed in the face phase
-    R vn[NS ? VT : 1];
+    constexpr int VW = NS ? vis_width<R>() : 1;
+    R vn[VW];
     R invh = R(0);
     if (NS && face_active) {
         if ((fr.x & 15) <= FK_PERIODIC) {
-#pragma unroll
-            for (int c = 0; c < (NS ? VT : 1); ++c) vn[c] = (R)((const TR *)a.dtr)[nslot * VT + c];
+            load_viscous_trace<R, TR>(a, nslot, nx, ny, (fr.x & 15) == FK_PERIODIC, vn);
             if (XB && a.mu_a && (fr.x & 15) == FK_PERIODIC) {
                 // a periodic face is a boundary edge of each side, whose viscosity (its own
                 // element's mu_a) both sides' fluxes take; the partner stored its trace with its own
                 const double ms = a.ph.mu + a.mu_a[fe], mp = a.ph.mu + a.mu_a[fr.y >> 2];
                 const R sc = (R)(ms / mp);
 #pragma unroll
-                for (int c = 0; c < (NS ? VT : 1); ++c) vn[c] = vn[c] * sc;
+                for (int c = 0; c < VW; ++c) vn[c] = vn[c] * sc;
             }
         }
         if (IP) invh = (R)a.einvh[fr.w];
@@ -1078,12 +1106,8 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                 FaceV::put(sV, t, gc);
             }
         } else {
-            R vs[NS ? VT : 1];   // own viscous flux trace
-            if (NS) {
-                const TR *vt = (const TR *)a.dtr + ((int64_t)(fe * 4 + ff) * P + fk) * VT;
-#pragma unroll
-                for (int c = 0; c < (NS ? VT : 1); ++c) vs[c] = (R)vt[c];
-            }
+            R vs[VW];   // own viscous flux trace
+            if (NS) load_viscous_trace<R, TR>(a, (int64_t)(fe * 4 + ff) * P + fk, nx, ny, false, vs);
             int rs = a.ph.riemann;
             R uSB[4] = {R(0), R(0), R(0), R(0)};
             int neumann = 0, prescribed = 0;
@@ -1116,16 +1140,21 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                 const R pen = IP ? ph.sigma0 * muf * (R)(P - 1) * (R)(P - 1) * invh : R(0);
                 if (kind <= FK_PERIODIC) {
                     const R *uL = (kind == FK_INT_R) ? qo : qs, *uR = (kind == FK_INT_R) ? qs : qo;
-                    const R *vL = (kind == FK_INT_R) ? vn : vs, *vR = (kind == FK_INT_R) ? vs : vn;
-                    R fL[4], gL[4], fR[4], gR[4];
-                    viscous_trace_flux(vL, fL, gL);
-                    viscous_trace_flux(vR, fR, gR);
+                    if constexpr (sizeof(R) == 8) {
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        R acc = R(0);
-                        acc = acc + R(0.5) * (fL[c] + fR[c]) * nx;
-                        acc = acc + R(0.5) * (gL[c] + gR[c]) * ny;
-                        Fv[c] = acc;
+                        for (int c = 0; c < VW; ++c) Fv[c + 1] = R(0.5) * (vs[c] + vn[c]);
+                    } else {
+                        const R *vL = (kind == FK_INT_R) ? vn : vs, *vR = (kind == FK_INT_R) ? vs : vn;
+                        R fL[4], gL[4], fR[4], gR[4];
+                        viscous_trace_flux(vL, fL, gL);
+                        viscous_trace_flux(vR, fR, gR);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            R acc = R(0);
+                            acc = acc + R(0.5) * (fL[c] + fR[c]) * nx;
+                            acc = acc + R(0.5) * (gL[c] + gR[c]) * ny;
+                            Fv[c] = acc;
+                        }
                     }
                     if (IP) {
 #pragma unroll
@@ -1148,14 +1177,20 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                     }
                 } else if (!neumann) {
                     const bool adiab = is_adiabatic(fr.x);
-                    R fv4[4], gv4[4];
-                    viscous_trace_flux(vs, fv4, gv4);   // adiabatic or not, as the gradient kernel chose
+                    // adiabatic or not, as the gradient kernel chose
+                    if constexpr (sizeof(R) == 8) {
 #pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        R acc = R(0);
-                        acc = acc + fv4[c] * nx;
-                        acc = acc + gv4[c] * ny;
-                        Fv[c] = acc;
+                        for (int c = 0; c < VW; ++c) Fv[c + 1] = vs[c];
+                    } else {
+                        R fv4[4], gv4[4];
+                        viscous_trace_flux(vs, fv4, gv4);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            R acc = R(0);
+                            acc = acc + fv4[c] * nx;
+                            acc = acc + gv4[c] * ny;
+                            Fv[c] = acc;
+                        }
                     }
                     if (IP) {
 #pragma unroll
@@ -1354,7 +1389,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
                     for (int c = 0; c < 8; ++c) ds[c] *= mij;
                     const int64_t slot = (int64_t)(fe * 4 + ff) * P + fk;
                     double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + slot * 8 : nullptr;
-                    put_viscous_trace<double, double>(ph, fr.x, qn, ds, (double *)a.dtr_out + slot * VT, ph.mu, mdq);
+                    put_viscous_trace<double, double>(a, ph, fr.x, qn, ds, slot, nx, ny, ph.mu, mdq);
                 }
                 return;
             }
@@ -1391,9 +1426,10 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             }
             __syncthreads();
             if (face_active) {
-                double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + ((int64_t)(fe * 4 + ff) * P + fk) * 8 : nullptr;
-                viscous_face_trace<P, NL, R, TR, UNROLL>(a, ph, fr.x, qn, sDQ, fs * Layout<P>::ES, sLb, sLbw + 2 * P, ff, fk,
-                                                (TR *)a.dtr_out + ((int64_t)(fe * 4 + ff) * P + fk) * VT, ph.mu, mdq);
+                const int64_t slot = (int64_t)(fe * 4 + ff) * P + fk;
+                double *mdq = ((fr.x & 15) == FK_MORTAR && a.mdq) ? a.mdq + slot * 8 : nullptr;
+                viscous_face_trace<P, NL, R, TR, UNROLL>(a, ph, fr.x, qn, sDQ, fs * Layout<P>::ES, sLb, sLbw + 2 * P, ff,
+                                                         fk, slot, nx, ny, ph.mu, mdq);
             }
           }
         }

@@ -46,3 +46,30 @@ def test_constant_metric_matches_oracle(N, viscous, kind):
         dg.rk_step(0.0, dt)
     ref = orc.state()
     assert np.max(np.abs(dg.state() - ref)) <= 1e-12 * np.max(np.abs(ref))
+
+
+@pytest.mark.parametrize("slant", [0.0, 0.15])
+@pytest.mark.parametrize("N", [2, 5, 6])
+@pytest.mark.parametrize("viscous", ["br1", "ip"])
+def test_periodic_viscous_trace_matches_oracle(N, viscous, slant):
+    """Viscous traces stored along the normal, and per direction where a periodic pair (matched by one
+    coordinate of its ends) is not parallel: both within the FP64 bar."""
+    from horses2d_amd import gpu
+    from oracle.oracle import Oracle
+    wall = C.Zone(C.BC_VISCOUSWALL)
+    mesh = C.channel(6, 5, 2.0, 1.0, [wall, C.Zone(C.BC_PERIODIC, direction=1, partner=4), wall,
+                                      C.Zone(C.BC_PERIODIC, direction=1, partner=2)])
+    mesh.points[:, 0] *= 1.0 + slant * mesh.points[:, 1]
+    case = C.Case("slanted", mesh, np.full(mesh.K, N, np.int32), 0.3, 200.0, 0.72, True, riemann="roe",
+                  viscous=viscous, cfl=0.05, ic=C.isentropic_vortex(0.3, 1.0, 1.0, 0.5))
+    orc = Oracle(case)
+    Q0 = case.initial_state(orc.coords())
+    orc.set_state(Q0)
+    dt = orc.estimate_dt(case.dt_max, case.cfl)
+    dg = gpu.DGSEM(case, "fp64", apply_ic=False)
+    dg.upload(Q0)
+    for _ in range(3):
+        orc.step(0.0, dt, case.scheme)
+        dg.rk_step(0.0, dt)
+    ref = orc.state()
+    assert np.max(np.abs(dg.state() - ref)) <= 1e-12 * np.max(np.abs(ref))
