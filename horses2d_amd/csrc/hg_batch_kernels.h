@@ -59,7 +59,7 @@ __device__ inline int4 uniform_item(const int4 *__restrict__ items, const int *_
 }
 
 template <int TILE, bool NS, bool IP, int RS, typename R, typename TR>
-__global__ __launch_bounds__(256) void k_batch_stage(const StageArgs *__restrict__ slots, const int4 *__restrict__ items,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, RS, false, sizeof(R) == 8)))) void k_batch_stage(const StageArgs *__restrict__ slots, const int4 *__restrict__ items,
                                                      const int *__restrict__ sched, const double *__restrict__ dt,
                                                      BatchArgs b) {
     __shared__ BatchStageSmem<TILE, NS, IP, R> S;
@@ -274,7 +274,8 @@ hipError_t persist_grid(K kernel, int block, const BatchArgs &b, PersistGrid &g,
 // register count of the costliest order for every item).  Same stage_body / gradient_body, so
 // the same bits.
 template <int P, int TILE, bool NS, bool IP, int RS, typename R, typename TR>
-__global__ __launch_bounds__((Tile<P, TileOf<P, TILE>::EPB>::TPB)) void k_batch_stage_p(
+__global__ __launch_bounds__((Tile<P, TileOf<P, TILE>::EPB>::TPB))
+    __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, RS, false, sizeof(R) == 8)))) void k_batch_stage_p(
     const StageArgs *__restrict__ slots, const int4 *__restrict__ items, const int *__restrict__ sched,
     const double *__restrict__ dt, BatchArgs b) {
     constexpr int EPB = TileOf<P, TILE>::EPB;

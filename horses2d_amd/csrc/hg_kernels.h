@@ -911,17 +911,23 @@ struct StageSmem {
     // U / V lift coefficients.  FP64: the flux along the face in sU, then V there, while U, whose
     // weight is the face flux's, is added to sF: the fifth of the LDS this saves lets four workgroups
     // instead of three share a CU (P = 4 to 7; 101 x 77, N = 5: 28.5 -> 25.6 us a stage).
-    alignas(16) R sU[IP ? T::NF * 4 : 1];
-    alignas(16) R sV[IP && sizeof(R) == 4 ? T::NF * 4 : 1];
+    alignas(16) R sU[IP ? T::NF * 4 : NS ? 1 : 0];
+    alignas(16) R sV[IP && sizeof(R) == 4 ? T::NF * 4 : NS ? 1 : 0];
     alignas(16) R sHat[T::PP];          // transposed, as sD: a wavefront's reads are consecutive
-    alignas(16) R sD[NS ? T::PP : 1];   // IP gradient; BR1: the Laplacian dissipation's interior gradient
-    alignas(16) R sLbw[IP && sizeof(R) == 4 ? 4 * P : 2 * P];   // lbw; IP in FP32: lb (epilogue) behind it
-    alignas(16) R sDlbw[2 * P];
+    alignas(16) R sD[NS ? T::PP : 0];   // IP gradient; BR1: the Laplacian dissipation's interior gradient
+    // Euler in FP64 reads lbw from memory and holds nothing it does not need: LDS is allocated in 1280
+    // bytes, and at P = 6 to 8 it is at 25 of these that five workgroups share a CU's 160 KB (64 cases
+    // of N = 3 to 8 in one launch: 3197 -> 2758 us a step; 128 x 128, N = 7: 38.4 -> 37.3 us a stage)
+    alignas(16) R sLbw[IP && sizeof(R) == 4 ? 4 * P : NS || sizeof(R) == 4 ? 2 * P : 0];   // lbw; IP in FP32: lb (epilogue) behind it
+    alignas(16) R sDlbw[NS ? 2 * P : 0];
 };
 
-// Wavefronts per SIMD the stage kernel's register allocation has to leave room for: four of the FP64
-// Navier-Stokes form with one solver (P = 8, interior penalty: 129 registers without it).
-constexpr int stage_waves(bool ns, bool one_solver, bool fp64) { return ns && one_solver && fp64 ? 4 : 1; }
+// Wavefronts per SIMD the stage kernel's register allocation has to leave room for: in FP64, as many as
+// the wide tiles' LDS allows, four of the Navier-Stokes form with one solver and five of the Euler form
+// (but for the exact solver, which needs 135 registers).
+constexpr int stage_waves(bool ns, int rs, bool xbf, bool fp64) {
+    return !fp64 || rs < 0 || xbf ? 1 : ns ? 4 : rs == 2 ? 1 : 5;
+}
 
 // One element tile [e0, e0+EPB) of a stage; any workgroup size >= Tile<P, EPB>::TPB (at most
 // 256).  rslot is the residual partial this tile writes; cq, cg are the stage's RK factors.
@@ -945,6 +951,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     // compiled in, and FP32 interior penalty, are where the registers this takes cost a wavefront per SIMD
     // (256 x 256, N = 7, mixed: 78 registers and 543 us a step at 2, 81 and 575 us unrolled).
     constexpr int UNROLL = (XB || RS == 2) ? 1 : (IP && sizeof(R) == 4) ? 2 : P;
+    constexpr bool LBW_MEM = !NS && sizeof(R) == 8;
     const int TPB = blockDim.x;
     double *sQ = S.sQ, *sLb = S.sLb;
     R *sCF = S.u.f.sCF, *sCG = S.u.f.sCG, *sF = S.sF, *sU = S.sU, *sV = S.sV;
@@ -955,7 +962,9 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
     const bool affine = NS && sizeof(R) == 8 && a.affine;   // constant metric
     if (a.resid_max && !a.do_resid && e0 == 0 && t < 4) a.resid_max[t * kResidStride] = 0.0;
     if (t < 2 * P) {
-        sLb[t] = a.lb[t]; sLbw[t] = (R)a.lbw[t]; sDlbw[t] = (R)a.dlbw[t];
+        sLb[t] = a.lb[t];
+        if (!LBW_MEM) sLbw[t] = (R)a.lbw[t];
+        if (NS) sDlbw[t] = (R)a.dlbw[t];
         if (IP && sizeof(R) == 4) sLbw[2 * P + t] = (R)a.lb[t];
     }
     for (int x = t; x < PP; x += TPB) {
@@ -1314,7 +1323,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
             const int idx = (f == 0 || f == 2) ? i : j;
             const int oth = (f == 0 || f == 2) ? j : i;
             const int side = (f == 0 || f == 3) ? 0 : P;
-            const R lw = sLbw[side + oth];
+            const R lw = LBW_MEM ? (R)a.lbw[side + oth] : sLbw[side + oth];
             const int xf = (s * 4 + f) * P + idx;
             R Ff[4];
             FaceV::get(sF, xf, Ff);
@@ -1464,7 +1473,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
 
 template <int P, int EPB, bool NS, bool IP, int RS, typename R, typename TR, bool XBF = false>
 __global__ __launch_bounds__((Tile<P, EPB>::TPB))
-    __attribute__((amdgpu_waves_per_eu(stage_waves(NS, RS >= 0 && !XBF, sizeof(R) == 8)))) void k_stage(StageArgs a) {
+    __attribute__((amdgpu_waves_per_eu(stage_waves(NS, RS, XBF, sizeof(R) == 8)))) void k_stage(StageArgs a) {
     __shared__ StageSmem<P, EPB, NS, IP, R> S;
     double cq = a.cq, cg = a.cg;
     if (a.dt_dev) {   // graph replay: the step size lives in device memory
