@@ -179,14 +179,15 @@ __device__ inline int persist_order(const PersistGrid &g, int w, int &r) {
     case PV: CALL(PV, p##PV); break;
 
 // The FP32 form keeps the occupancy of the one-item kernel (eight wavefronts per SIMD, 64
-// VGPRs): without the bound the loop's hoisted lane-index values take it to 86 VGPRs.
+// VGPRs): without the bound the loop's hoisted lane-index values take it to 86 VGPRs.  The FP64 Euler
+// form to four: 137 VGPRs without (64 cases of N = 3 to 8: 4049 -> 3936 us a step).
 template <typename R>
-struct PersistWaves {
-    static constexpr int value = sizeof(R) == 4 ? 8 : 1;
-};
+constexpr int persist_waves(bool ns, int rs) {
+    return sizeof(R) == 4 ? 8 : stage_waves(ns, rs, false, true) == 5 ? 4 : 1;
+}
 
 template <int TILE, bool NS, bool IP, int RS, typename R, typename TR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(PersistWaves<R>::value))) void k_batch_stage_persist(const StageArgs *__restrict__ slots,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(persist_waves<R>(NS, RS)))) void k_batch_stage_persist(const StageArgs *__restrict__ slots,
                                                              const int4 *__restrict__ items,
                                                              const double *__restrict__ dt, BatchArgs b,
                                                              PersistGrid g) {
