@@ -73,8 +73,9 @@ hipError_t take_set(int device, Staging **out) {
     s->device = device;
     hipError_t e = hipSuccess;
     for (int b = 0; b < 2 && e == hipSuccess; ++b) {
-        e = hipHostMalloc(&s->buf[b], kBuffer, hipHostMallocPortable);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&s->done[b], hipEventDisableTiming);
+        // kernels write these buffers and the host reads them after the event
+        e = hipHostMalloc(&s->buf[b], kBuffer, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&s->done[b], hipEventDisableTiming | hipEventReleaseToSystem);
     }
     if (e != hipSuccess) {
         release_set(s);

@@ -1,0 +1,58 @@
+"""What the host side asks of the HIP runtime when it moves data, on a stand-in for it (fake_hip.c, which
+needs no GPU): each test runs a child process that loads the stand-in before the library."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRELUDE = """
+import ctypes, sys, threading
+import numpy as np
+F = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
+F.fake_host_flags.restype = F.fake_event_flags.restype = ctypes.c_uint
+F.fake_count.restype = F.fake_pending.restype = ctypes.c_long
+F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
+F.fake_pinned_most.restype = ctypes.c_size_t
+sys.path.insert(0, {root!r})
+from horses2d_amd import gpu, cases as C
+HOST_MALLOC, EVENT_CREATE, EVENT_RECORD, EVENT_SYNC, STREAM_SYNC, COPY_ASYNC, LAUNCH = range(7)
+
+def solver(nx, ny, N, precision="fp64"):
+    mesh = C.periodic_rectangle(nx, ny, -5.0, 5.0, -5.0, 5.0)
+    return gpu.DGSEM(C.Case("t", mesh, np.full(mesh.K, N, np.int32), 0.5, cfl=0.1), precision, apply_ic=False)
+
+def values(dg, seed):
+    q = np.random.Generator(np.random.PCG64(seed)).uniform(0.5, 1.5, dg.ndof)
+    q.reshape(-1, 4)[:, 3] += 3.0
+    return q
+"""
+
+
+@pytest.fixture(scope="module")
+def child(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "fake_hip.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", "-o", so, os.path.join(HERE, "fake_hip.c"), "-lpthread"],
+                   check=True)
+
+    def run(code):
+        r = subprocess.run([sys.executable, "-c", PRELUDE.format(so=so, root=os.path.dirname(HERE)) + code],
+                           capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout + r.stderr
+    return run
+
+
+def test_staging_memory_is_coherent_by_contract(child):
+    """Kernels write the staging buffers and the host reads them after an event: coherent memory
+    (hipHostMallocCoherent) and events that release to the system (hipEventReleaseToSystem), whatever the
+    environment's defaults."""
+    child("""
+dg = solver(16, 16, 4)
+q = values(dg, 1)
+dg.upload(q)
+assert (dg.state() == q).all()
+assert F.fake_count(HOST_MALLOC) > 0 and F.fake_count(EVENT_CREATE) > 0
+assert F.fake_host_flags() & 0x40000000, hex(F.fake_host_flags())
+assert F.fake_event_flags() & 0x80000000, hex(F.fake_event_flags())
+""")
