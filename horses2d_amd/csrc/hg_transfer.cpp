@@ -97,10 +97,19 @@ void give_set(Staging *s) {
     release_set(s);
 }
 
+// After a failed transfer: whatever it left on the stream may still use the buffers, and no event
+// marks its end, so the set does not go back to the pool.
+void discard_set(Staging *s, hipStream_t stream) {
+    if (!s) return;
+    (void)hipStreamSynchronize(stream);
+    release_set(s);
+}
+
 hipError_t wait_buffer(Staging *s, int b) {
     if (!s->used[b]) return hipSuccess;
-    s->used[b] = false;
-    return hipEventSynchronize(s->done[b]);
+    const hipError_t e = hipEventSynchronize(s->done[b]);
+    if (e == hipSuccess) s->used[b] = false;
+    return e;
 }
 
 // Makes the handle's device current in the calling thread, and back again.
@@ -130,7 +139,7 @@ hipError_t move_share(int device, hipStream_t stream, char *host, char *dev, siz
         const int b = (int)(k & 1);
         if (k < n) {
             e = wait_buffer(s, b);
-            if (to_dev) std::memcpy(s->buf[b], host + k * chunk, len(k));
+            if (to_dev && e == hipSuccess) std::memcpy(s->buf[b], host + k * chunk, len(k));
             if (e == hipSuccess)
                 e = n <= kByKernel && len(k) % 16 == 0
                         ? hg::launch_copy(to_dev ? s->buf[b] : dev + k * chunk, to_dev ? dev + k * chunk : s->buf[b],
@@ -138,7 +147,7 @@ hipError_t move_share(int device, hipStream_t stream, char *host, char *dev, siz
                     : to_dev ? hipMemcpyAsync(dev + k * chunk, s->buf[b], len(k), hipMemcpyHostToDevice, stream)
                              : hipMemcpyAsync(s->buf[b], dev + k * chunk, len(k), hipMemcpyDeviceToHost, stream);
             if (e == hipSuccess) e = hipEventRecord(s->done[b], stream);
-            s->used[b] = e == hipSuccess;
+            if (e == hipSuccess) s->used[b] = true;
         }
         if (!to_dev && k > 0 && e == hipSuccess) {
             // the chunk before, while this one's transfer runs
@@ -146,7 +155,8 @@ hipError_t move_share(int device, hipStream_t stream, char *host, char *dev, siz
             if (e == hipSuccess) std::memcpy(host + (k - 1) * chunk, s->buf[b ^ 1], len(k - 1));
         }
     }
-    give_set(s);   // a buffer whose upload still runs is waited for by its next user
+    if (e == hipSuccess) give_set(s);   // a buffer whose upload still runs is waited for by its next user
+    else discard_set(s, stream);
     return e;
 }
 
@@ -239,8 +249,12 @@ hipError_t read_values(hg_handle *h, double *dst, const double *src, int n, int 
     e = wait_buffer(s, 0);
     if (e == hipSuccess) e = launch_store_values(src, n, stride, (double *)s->buf[0], h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);
-    if (e == hipSuccess) std::memcpy(dst, s->buf[0], n * sizeof(double));
-    give_set(s);
+    if (e == hipSuccess) {
+        std::memcpy(dst, s->buf[0], n * sizeof(double));
+        give_set(s);
+    } else {
+        discard_set(s, h->stream);
+    }
     return e;
 }
 

@@ -56,3 +56,44 @@ assert F.fake_count(HOST_MALLOC) > 0 and F.fake_count(EVENT_CREATE) > 0
 assert F.fake_host_flags() & 0x40000000, hex(F.fake_host_flags())
 assert F.fake_event_flags() & 0x80000000, hex(F.fake_event_flags())
 """)
+
+
+@pytest.mark.parametrize("what, left", [("EVENT_RECORD", "a.state()"), ("STREAM_SYNC", "a.residuals()"),
+                                        ("EVENT_SYNC", "a.state()")])
+def test_failed_read_leaves_the_pool_clean(child, what, left):
+    """A read of one handle that fails with its transfer still on the stream does not hand the buffer that
+    transfer writes to another handle."""
+    child(f"""
+a, b = solver(16, 16, 4), solver(16, 16, 4)
+qa, qb = values(a, 1), values(b, 2)
+a.upload(qa); b.upload(qb)
+assert (a.state() == qa).all() and (b.state() == qb).all()
+F.fake_fail({what}, 1)
+try:
+    {left}
+except RuntimeError:
+    pass
+else:
+    raise SystemExit("the failure was not reported")
+F.fake_fail({what}, 0)
+assert (b.state() == qb).all()
+assert (a.state() == qa).all()
+""")
+
+
+def test_failed_upload_leaves_the_one_before_it(child):
+    """An upload that cannot wait for the buffer's last transfer does not write into the buffer."""
+    child("""
+a, b = solver(16, 16, 4), solver(16, 16, 4)
+qa, qb = values(a, 1), values(b, 2)
+a.upload(qa)
+F.fake_fail(EVENT_SYNC, 1)
+try:
+    b.upload(qb)
+except RuntimeError:
+    pass
+F.fake_fail(EVENT_SYNC, 0)
+assert (a.state() == qa).all()
+b.upload(qb)
+assert (b.state() == qb).all()
+""")
