@@ -18,6 +18,7 @@
 #include <exception>
 #include <functional>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -59,30 +60,32 @@ void release_set(Staging *s) {
     delete s;
 }
 
-hipError_t take_set(int device, Staging **out) {
+// A set for a device (current in this thread); null where pinned memory or an event is not to be had.
+Staging *take_set(int device) {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         for (size_t k = g_idle.size(); k-- > 0;)
             if (g_idle[k]->device == device) {
-                *out = g_idle[k];
+                Staging *s = g_idle[k];
                 g_idle.erase(g_idle.begin() + (long)k);
-                return hipSuccess;
+                return s;
             }
     }
-    Staging *s = new Staging();
+    Staging *s = new (std::nothrow) Staging();
+    if (!s) return nullptr;
     s->device = device;
     hipError_t e = hipSuccess;
     for (int b = 0; b < 2 && e == hipSuccess; ++b) {
         // kernels write these buffers and the host reads them after the event
         e = hipHostMalloc(&s->buf[b], kBuffer, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&s->done[b], hipEventDisableTiming | hipEventReleaseToSystem);
+        else s->buf[b] = nullptr;
+        if (e != hipSuccess) s->done[b] = nullptr;
     }
-    if (e != hipSuccess) {
-        release_set(s);
-        s = nullptr;
-    }
-    *out = s;
-    return e;
+    if (e == hipSuccess) return s;
+    release_set(s);
+    (void)hipGetLastError();   // the caller goes another way
+    return nullptr;
 }
 
 void give_set(Staging *s) {
@@ -98,11 +101,12 @@ void give_set(Staging *s) {
 }
 
 // After a failed transfer: whatever it left on the stream may still use the buffers, and no event
-// marks its end, so the set does not go back to the pool.
+// marks its end, so the set does not go back to the pool.  The caller reports the error; it does not
+// stay for the next launch's hipGetLastError.
 void discard_set(Staging *s, hipStream_t stream) {
-    if (!s) return;
     (void)hipStreamSynchronize(stream);
     release_set(s);
+    (void)hipGetLastError();
 }
 
 hipError_t wait_buffer(Staging *s, int b) {
@@ -126,13 +130,17 @@ struct OnDevice {
     }
 };
 
-// One share, between host and dev.
+// One share, between host and dev; without a staging set, by the runtime's own path.
 hipError_t move_share(int device, hipStream_t stream, char *host, char *dev, size_t bytes, bool to_dev) {
     OnDevice on(device);
     hipError_t e = on.err;
-    Staging *s = nullptr;
-    if (e == hipSuccess) e = take_set(device, &s);
     if (e != hipSuccess) return e;
+    Staging *s = take_set(device);
+    if (!s) {
+        e = to_dev ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, stream)
+                   : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream);
+        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
+    }
     const size_t chunk = bytes < kShare ? kShort : bytes < kLong ? kBuffer / 2 : kBuffer, n = (bytes + chunk - 1) / chunk;
     auto len = [&](size_t k) { return std::min(chunk, bytes - k * chunk); };
     for (size_t k = 0; k < n + (to_dev ? 0 : 1) && e == hipSuccess; ++k) {
@@ -239,13 +247,15 @@ hipError_t read_values(hg_handle *h, double *dst, const double *src, int n, int 
     if ((size_t)n * sizeof(double) > kBuffer) return hipErrorInvalidValue;
     OnDevice on(h->device);
     hipError_t e = on.err;
-    Staging *s = nullptr;
-    try {
-        if (e == hipSuccess) e = take_set(h->device, &s);
-    } catch (const std::exception &) {
-        e = hipErrorOutOfMemory;
-    }
     if (e != hipSuccess) return e;
+    Staging *s = take_set(h->device);
+    if (!s) {
+        const int m = stride == 1 ? 1 : n;   // copies
+        for (int i = 0; i < m && e == hipSuccess; ++i)
+            e = hipMemcpyAsync(dst + i, src + (int64_t)i * stride, (n / m) * sizeof(double), hipMemcpyDeviceToHost,
+                               h->stream);
+        return e == hipSuccess ? hipStreamSynchronize(h->stream) : e;
+    }
     e = wait_buffer(s, 0);
     if (e == hipSuccess) e = launch_store_values(src, n, stride, (double *)s->buf[0], h->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(h->stream);

@@ -46,9 +46,12 @@ long fake_pending(void) {
     return n;
 }
 
+enum { FAILED = 999 };
+static __thread int last_error;   /* stays until hipGetLastError reads it */
 static int bad(int k) {   /* mu held */
     const long c = ++count[k], f = fail_at[k];
-    return f < 0 || (f > 0 && c == f);
+    if (!(f < 0 || (f > 0 && c == f))) return 0;
+    return last_error = FAILED;
 }
 
 static void run(stream *s, long upto) {
@@ -77,13 +80,16 @@ static void queue(stream *s, void *dst, const void *src, size_t n) {
 }
 #define IN pthread_mutex_lock(&mu)
 #define OUT(x) do { const int r_ = (x); pthread_mutex_unlock(&mu); return r_; } while (0)
-enum { FAILED = 999 };
 
 int hipGetDevice(int *d) { *d = 0; return 0; }
 int hipSetDevice(int d) { (void)d; return 0; }
 int hipGetDeviceCount(int *n) { *n = 1; return 0; }
 int hipDeviceGetAttribute(int *v, int a, int d) { (void)a; (void)d; *v = 256; return 0; }
-int hipGetLastError(void) { return 0; }
+int hipGetLastError(void) {
+    const int e = last_error;
+    last_error = 0;
+    return e;
+}
 const char *hipGetErrorString(int e) { (void)e; return "made to fail"; }
 int hipMalloc(void **p, size_t n) { *p = calloc(1, n + 64); return *p ? 0 : 2; }
 int hipFree(void *p) { free(p); return 0; }

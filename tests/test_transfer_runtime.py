@@ -97,3 +97,20 @@ assert (a.state() == qa).all()
 b.upload(qb)
 assert (b.state() == qb).all()
 """)
+
+
+@pytest.mark.parametrize("what", ["HOST_MALLOC", "EVENT_CREATE"])
+@pytest.mark.parametrize("nx, N", [(16, 4), (80, 5), (200, 6)])
+def test_transfers_without_pinned_memory(child, nx, N, what):
+    """Where pinned memory (or an event) is not to be had, the runtime's own path moves the data."""
+    child(f"""
+dg = solver({nx}, {nx}, {N})
+q = values(dg, 1)
+F.fake_fail({what}, -1)
+dg.upload(q)
+assert (dg.state() == q).all()
+assert (dg.residuals() == 0.0).all() and dg.conservation_sums().shape == (4,)
+F.fake_fail({what}, 0)
+dg.upload(2.0 * q)
+assert (dg.state() == 2.0 * q).all()
+""")
