@@ -5,7 +5,6 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
-#include <exception>
 #include <memory>
 #include <mutex>
 #include <numeric>
@@ -1248,23 +1247,12 @@ int hg_build_geometry(const hg_mesh_desc *mesh, int64_t nnodes, double *X, doubl
     return 0;
 }
 
-// The mean nodal pressure of a state (0 when it is not finite).  The divisions are shared out, the
-// sum runs over the nodes in order: the FP32 form's rounding follows every bit of this value.
+// The mean nodal pressure of a state (0 when it is not finite).
 static double mean_pressure(double gm1, const double *Q, int64_t nodes) {
-    auto pressure = [&](int64_t n) {
-        const double *q = Q + 4 * n;
-        return gm1 * (q[3] - 0.5 * (q[1] * q[1] + q[2] * q[2]) / q[0]);
-    };
     double sum = 0.0;
-    try {
-        std::vector<double> p(nodes);
-        hg::in_shares(nodes, 65536, [&](int64_t n0, int64_t n1) {
-            for (int64_t n = n0; n < n1; ++n) p[n] = pressure(n);
-        });
-        for (double v : p) sum += v;
-    } catch (const std::exception &) {   // no memory for them
-        sum = 0.0;
-        for (int64_t n = 0; n < nodes; ++n) sum += pressure(n);
+    for (int64_t n = 0; n < nodes; ++n) {
+        const double *q = Q + 4 * n;
+        sum += gm1 * (q[3] - 0.5 * (q[1] * q[1] + q[2] * q[2]) / q[0]);
     }
     const double pref = nodes > 0 ? sum / (double)nodes : 0.0;
     return std::isfinite(pref) ? pref : 0.0;

@@ -14,7 +14,7 @@ F = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
 F.fake_host_flags.restype = F.fake_event_flags.restype = ctypes.c_uint
 F.fake_count.restype = F.fake_pending.restype = ctypes.c_long
 F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
-F.fake_pinned_most.restype = ctypes.c_size_t
+F.fake_pinned_most.restype = F.fake_largest_new.restype = ctypes.c_size_t
 sys.path.insert(0, {root!r})
 from horses2d_amd import gpu, cases as C
 HOST_MALLOC, EVENT_CREATE, EVENT_RECORD, EVENT_SYNC, STREAM_SYNC, COPY_ASYNC, LAUNCH = range(7)
@@ -113,4 +113,17 @@ assert (dg.residuals() == 0.0).all() and dg.conservation_sums().shape == (4,)
 F.fake_fail({what}, 0)
 dg.upload(2.0 * q)
 assert (dg.state() == 2.0 * q).all()
+""")
+
+
+def test_upload_of_the_mixed_form_needs_no_memory_of_its_own(child):
+    """The mixed form's reference pressure is summed while the state is read: an array of the nodes'
+    pressures cost a fifth of the upload's time at 90 k nodes (239 us against 195)."""
+    child("""
+dg = solver(60, 60, 4, "mixed")
+q = values(dg, 1)
+F.fake_largest_new()
+dg.upload(q)
+assert F.fake_largest_new() < 8 * dg.nodes
+assert (dg.state() == q).all()
 """)
