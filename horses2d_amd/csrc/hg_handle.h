@@ -4,7 +4,6 @@
 
 #include <algorithm>
 #include <cstdint>
-#include <functional>
 #include <string>
 #include <utility>
 #include <vector>
@@ -167,8 +166,6 @@ int handle_error(const std::string &m);
 hipError_t copy_to_host(hg_handle *h, void *dst, const void *src, size_t bytes);
 hipError_t copy_to_device(hg_handle *h, void *dst, const void *src, size_t bytes);
 hipError_t read_values(hg_handle *h, double *dst, const double *src, int n, int stride = 1);
-// f(first, last) over [0, n) in contiguous shares of at least `least`, on up to four threads.
-void in_shares(int64_t n, int64_t least, const std::function<void(int64_t, int64_t)> &f);
 void transfers_open();
 void transfers_close();
 // Locates the allocation-free entry points' scratch array on a device (once per device).

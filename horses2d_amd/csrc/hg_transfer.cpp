@@ -8,15 +8,15 @@
 // a kernel, without the copy engine's start and signals (205 kB: 21 us, four values 14 us).  Uploads are
 // staged up to a MiB; the runtime maps longer arrays in place, at 30 GB/s.
 //
-// The staging sets belong to a process-wide pool: a set is taken for one share of one transfer, at
-// most kIdleSets are kept, and the last handle's destruction frees them.
+// The staging sets belong to a process-wide pool of at most kSets per device: a transfer takes what is
+// idle or may still be made, up to one per share, and goes the runtime's way when that is none.  The
+// last handle's destruction frees them.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <exception>
-#include <functional>
 #include <mutex>
 #include <new>
 #include <thread>
@@ -37,21 +37,23 @@ constexpr int kThreads = 4;
 // A share of at most this many chunks moves by a kernel that reads or writes the pinned buffer
 // itself, without the copy engine's start and its signals.
 constexpr size_t kByKernel = 2;
-constexpr size_t kIdleSets = 8;                  // 32 MiB of pinned memory
+// Sets of a device, 32 MiB of pinned memory.  Making one takes longer than a short transfer: with the sets
+// beyond eight freed after use, eight threads' states of 25.7 MB took 8.8 ms instead of the runtime's 5.2.
+constexpr int kSets = 8;
 
 struct Staging {
     int device = -1;
+    bool busy = true;                            // a transfer has it
     void *buf[2] = {nullptr, nullptr};
     hipEvent_t done[2] = {nullptr, nullptr};     // the last transfer of each buffer
     bool used[2] = {false, false};
 };
 
 std::mutex g_mutex;
-std::vector<Staging *> g_idle;
+std::vector<Staging *> g_sets;   // of every device
 int g_handles = 0;
 
 void release_set(Staging *s) {
-    if (!s) return;
     for (int b = 0; b < 2; ++b) {
         if (s->used[b]) (void)hipEventSynchronize(s->done[b]);
         if (s->done[b]) (void)hipEventDestroy(s->done[b]);
@@ -60,44 +62,68 @@ void release_set(Staging *s) {
     delete s;
 }
 
-// A set for a device (current in this thread); null where pinned memory or an event is not to be had.
-Staging *take_set(int device) {
+void drop_set(Staging *s) {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
-        for (size_t k = g_idle.size(); k-- > 0;)
-            if (g_idle[k]->device == device) {
-                Staging *s = g_idle[k];
-                g_idle.erase(g_idle.begin() + (long)k);
-                return s;
-            }
+        const auto at = std::find(g_sets.begin(), g_sets.end(), s);
+        if (at != g_sets.end()) g_sets.erase(at);
     }
-    Staging *s = new (std::nothrow) Staging();
-    if (!s) return nullptr;
-    s->device = device;
-    hipError_t e = hipSuccess;
-    for (int b = 0; b < 2 && e == hipSuccess; ++b) {
-        // kernels write these buffers and the host reads them after the event
-        e = hipHostMalloc(&s->buf[b], kBuffer, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent);
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&s->done[b], hipEventDisableTiming | hipEventReleaseToSystem);
-        else s->buf[b] = nullptr;
-        if (e != hipSuccess) s->done[b] = nullptr;
-    }
-    if (e == hipSuccess) return s;
     release_set(s);
-    (void)hipGetLastError();   // the caller goes another way
-    return nullptr;
+}
+
+bool make_buffers(Staging *s) {
+    for (int b = 0; b < 2; ++b) {
+        // kernels write these buffers and the host reads them after the event
+        if (hipHostMalloc(&s->buf[b], kBuffer, hipHostMallocPortable | hipHostMallocMapped | hipHostMallocCoherent) !=
+            hipSuccess) {
+            s->buf[b] = nullptr;
+            return false;
+        }
+        if (hipEventCreateWithFlags(&s->done[b], hipEventDisableTiming | hipEventReleaseToSystem) != hipSuccess) {
+            s->done[b] = nullptr;
+            return false;
+        }
+    }
+    return true;
+}
+
+// Up to `want` sets of a device (current in this thread); fewer, or none, where other transfers have them
+// or pinned memory or an event is not to be had.
+int take_sets(int device, int want, Staging **out) {
+    int got = 0, fresh;
+    {
+        std::lock_guard<std::mutex> lock(g_mutex);
+        int live = 0;
+        for (Staging *s : g_sets) {
+            if (s->device != device) continue;
+            ++live;
+            if (s->busy || got == want) continue;
+            s->busy = true;
+            out[got++] = s;
+        }
+        fresh = got;
+        try {
+            for (; got < want && live < kSets; ++live) {
+                g_sets.reserve(g_sets.size() + 1);
+                out[got] = new Staging();
+                out[got]->device = device;
+                g_sets.push_back(out[got++]);
+            }
+        } catch (const std::bad_alloc &) {   // what there is
+        }
+    }
+    for (int k = fresh; k < got; ++k)
+        if (!make_buffers(out[k])) {
+            (void)hipGetLastError();   // the caller goes another way
+            for (int j = k; j < got; ++j) drop_set(out[j]);
+            got = k;
+        }
+    return got;
 }
 
 void give_set(Staging *s) {
-    if (!s) return;
-    {
-        std::lock_guard<std::mutex> lock(g_mutex);
-        if (g_handles > 0 && g_idle.size() < kIdleSets) {
-            g_idle.push_back(s);
-            return;
-        }
-    }
-    release_set(s);
+    std::lock_guard<std::mutex> lock(g_mutex);
+    s->busy = false;
 }
 
 // After a failed transfer: whatever it left on the stream may still use the buffers, and no event
@@ -105,7 +131,7 @@ void give_set(Staging *s) {
 // stay for the next launch's hipGetLastError.
 void discard_set(Staging *s, hipStream_t stream) {
     (void)hipStreamSynchronize(stream);
-    release_set(s);
+    drop_set(s);
     (void)hipGetLastError();
 }
 
@@ -130,17 +156,10 @@ struct OnDevice {
     }
 };
 
-// One share, between host and dev; without a staging set, by the runtime's own path.
-hipError_t move_share(int device, hipStream_t stream, char *host, char *dev, size_t bytes, bool to_dev) {
-    OnDevice on(device);
+// One share, between host and dev, through a staging set.
+hipError_t move_share(Staging *s, hipStream_t stream, char *host, char *dev, size_t bytes, bool to_dev) {
+    OnDevice on(s->device);
     hipError_t e = on.err;
-    if (e != hipSuccess) return e;
-    Staging *s = take_set(device);
-    if (!s) {
-        e = to_dev ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, stream)
-                   : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, stream);
-        return e == hipSuccess ? hipStreamSynchronize(stream) : e;
-    }
     const size_t chunk = bytes < kShare ? kShort : bytes < kLong ? kBuffer / 2 : kBuffer, n = (bytes + chunk - 1) / chunk;
     auto len = [&](size_t k) { return std::min(chunk, bytes - k * chunk); };
     for (size_t k = 0; k < n + (to_dev ? 0 : 1) && e == hipSuccess; ++k) {
@@ -168,43 +187,42 @@ hipError_t move_share(int device, hipStream_t stream, char *host, char *dev, siz
     return e;
 }
 
+// By up to kThreads threads, one of them the caller's.
 hipError_t move(hg_handle *h, char *host, char *dev, size_t bytes, bool to_dev) {
+    if (bytes == 0) return hipSuccess;
+    OnDevice on(h->device);
+    if (on.err != hipSuccess) return on.err;
+    const size_t chunks = (bytes + kShort - 1) / kShort;
+    Staging *sets[kThreads];
+    const int want = (int)std::max<size_t>(1, std::min<size_t>(kThreads, chunks / (kShare / kShort)));
+    const int n = take_sets(h->device, want, sets);
+    if (n == 0) {
+        const hipError_t e = to_dev ? hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, h->stream)
+                                    : hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, h->stream);
+        return e == hipSuccess ? hipStreamSynchronize(h->stream) : e;
+    }
+    const size_t per = (chunks + n - 1) / n * kShort;
     std::atomic<int> err{(int)hipSuccess};
-    hg::in_shares((int64_t)((bytes + kShort - 1) / kShort), (int64_t)(kShare / kShort), [&](int64_t c0, int64_t c1) {
-        const size_t a = (size_t)c0 * kShort, b = std::min(bytes, (size_t)c1 * kShort);
-        hipError_t e = hipErrorOutOfMemory;
-        try {
-            e = move_share(h->device, h->stream, host + a, dev + a, b - a, to_dev);
-        } catch (const std::exception &) {
-        }
+    auto share = [&](int k) {
+        const size_t a = std::min(bytes, k * per), b = std::min(bytes, a + per);
+        const hipError_t e = move_share(sets[k], h->stream, host + a, dev + a, b - a, to_dev);
         if (e != hipSuccess) err = (int)e;
-    });
+    };
+    std::thread th[kThreads];
+    int k = n - 1;
+    try {
+        for (; k > 0; --k) th[k] = std::thread(share, k);
+    } catch (const std::exception &) {   // no more threads: the shares up to k are this one's
+    }
+    for (; k >= 0; --k) share(k);
+    for (std::thread &t : th)
+        if (t.joinable()) t.join();
     return (hipError_t)err.load();
 }
 
 }  // namespace
 
 namespace hg {
-
-void in_shares(int64_t n, int64_t least, const std::function<void(int64_t, int64_t)> &f) {
-    if (n <= 0) return;
-    const int64_t nt = std::max<int64_t>(1, std::min<int64_t>(kThreads, n / least)), per = (n + nt - 1) / nt;
-    std::vector<std::thread> th;
-    th.reserve((size_t)nt);
-    int64_t here = 0;   // the shares this thread does: [0, per), and those no thread was to be had for
-    for (int64_t k = nt - 1; k > 0; --k) {
-        const int64_t a = std::min(n, k * per), b = std::min(n, a + per);
-        if (a >= b) continue;
-        try {
-            th.emplace_back(std::cref(f), a, b);
-        } catch (const std::exception &) {
-            here = b;
-            break;
-        }
-    }
-    f(0, std::max(here, std::min(n, per)));
-    for (auto &t : th) t.join();
-}
 
 void transfers_open() {
     std::lock_guard<std::mutex> lock(g_mutex);
@@ -216,17 +234,13 @@ void transfers_close() {
     {
         std::lock_guard<std::mutex> lock(g_mutex);
         if (--g_handles > 0) return;
-        idle.swap(g_idle);
+        idle.swap(g_sets);
     }
     for (Staging *s : idle) release_set(s);
 }
 
 hipError_t copy_to_host(hg_handle *h, void *dst, const void *src, size_t bytes) {
-    try {
-        return move(h, (char *)dst, (char *)const_cast<void *>(src), bytes, false);
-    } catch (const std::exception &) {
-        return hipErrorOutOfMemory;
-    }
+    return move(h, (char *)dst, (char *)const_cast<void *>(src), bytes, false);
 }
 
 hipError_t copy_to_device(hg_handle *h, void *dst, const void *src, size_t bytes) {
@@ -234,11 +248,7 @@ hipError_t copy_to_device(hg_handle *h, void *dst, const void *src, size_t bytes
         const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream);
         return e == hipSuccess ? hipStreamSynchronize(h->stream) : e;
     }
-    try {
-        return move(h, (char *)const_cast<void *>(src), (char *)dst, bytes, true);
-    } catch (const std::exception &) {
-        return hipErrorOutOfMemory;
-    }
+    return move(h, (char *)const_cast<void *>(src), (char *)dst, bytes, true);
 }
 
 hipError_t read_values(hg_handle *h, double *dst, const double *src, int n, int stride) {
@@ -248,8 +258,8 @@ hipError_t read_values(hg_handle *h, double *dst, const double *src, int n, int 
     OnDevice on(h->device);
     hipError_t e = on.err;
     if (e != hipSuccess) return e;
-    Staging *s = take_set(h->device);
-    if (!s) {
+    Staging *s = nullptr;
+    if (!take_sets(h->device, 1, &s)) {
         const int m = stride == 1 ? 1 : n;   // copies
         for (int i = 0; i < m && e == hipSuccess; ++i)
             e = hipMemcpyAsync(dst + i, src + (int64_t)i * stride, (n / m) * sizeof(double), hipMemcpyDeviceToHost,

@@ -127,3 +127,27 @@ dg.upload(q)
 assert F.fake_largest_new() < 8 * dg.nodes
 assert (dg.state() == q).all()
 """)
+
+
+def test_many_threads_share_a_bounded_pool(child):
+    """Eight threads' reads, each of up to four shares, make at most eight staging sets (two buffers each)
+    in all and free none in between; whoever finds none goes the runtime's way."""
+    child("""
+solvers = [solver(100, 90 + k, 6) for k in range(8)]
+q = [values(s, k) for k, s in enumerate(solvers)]
+wrong = []
+def work(k):
+    solvers[k].upload(q[k])
+    for _ in range(6):
+        if not (solvers[k].state() == q[k]).all():
+            wrong.append(k)
+for _ in range(2):
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(8)]
+    [t.start() for t in threads]
+    [t.join() for t in threads]
+    assert not wrong
+    assert F.fake_count(HOST_MALLOC) <= 16 and F.fake_pinned_most() <= 32 << 20, F.fake_count(HOST_MALLOC)
+[s.close() for s in solvers]
+last = solver(16, 16, 4)
+assert (last.state() == 0.0).all() and F.fake_count(HOST_MALLOC) <= 18
+""")
