@@ -1302,6 +1302,7 @@ int hg_upload_state(hg_handle *h, const double *Q, int64_t ndof) {
     h->vtr_valid = false;
     h->qdot_valid = false;
     h->mon_tr = -1;
+    HG_CHECK(hipStreamSynchronize(h->stream));
     return 0;
 }
 

@@ -160,8 +160,8 @@ void mark_last_evaluation(hg_handle *h, int tr);
 // Records the message returned by hg_last_error and returns 1.
 int handle_error(const std::string &m);
 // Transfers through the process-wide pinned staging pool (hg_transfer.cpp), on the handle's stream.
-// copy_to_host returns with dst filled; copy_to_device with src free to change (the copy itself is
-// ordered on the stream).  read_values waits for the stream and returns src[i * stride], i < n.
+// copy_to_host returns with dst filled; copy_to_device is ordered on the stream, and src stays as it is
+// until the caller has waited for that.  read_values waits for the stream and returns src[i * stride], i < n.
 // Every handle opens the pool once and closes it when destroyed.
 hipError_t copy_to_host(hg_handle *h, void *dst, const void *src, size_t bytes);
 hipError_t copy_to_device(hg_handle *h, void *dst, const void *src, size_t bytes);

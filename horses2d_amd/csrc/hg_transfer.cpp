@@ -244,10 +244,7 @@ hipError_t copy_to_host(hg_handle *h, void *dst, const void *src, size_t bytes) 
 }
 
 hipError_t copy_to_device(hg_handle *h, void *dst, const void *src, size_t bytes) {
-    if (bytes > kByKernel * kShort) {
-        const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream);
-        return e == hipSuccess ? hipStreamSynchronize(h->stream) : e;
-    }
+    if (bytes > kByKernel * kShort) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, h->stream);
     return move(h, (char *)const_cast<void *>(src), (char *)dst, bytes, true);
 }
 

@@ -13,7 +13,7 @@
 
 typedef struct { uint32_t x, y, z; } dim3;
 typedef struct op { struct op *next; char *dst; const char *src; size_t n; long seq; } op;
-typedef struct stream { struct stream *next; op *head, *tail; } stream;
+typedef struct stream { struct stream *next; op *head, *tail; long unwaited; } stream;
 typedef struct { stream *s; long seq; unsigned flags; } event;
 typedef struct span { struct span *next; char *p; size_t n; } span;
 typedef struct fn { struct fn *next; const void *host; char name[256]; } fn;
@@ -32,6 +32,14 @@ static unsigned host_flags = ~0u, event_flags = ~0u;   /* the flags every such c
 static size_t pinned_now, pinned_most;
 
 long fake_count(int k) { return count[k]; }
+/* launches and copies of any stream since its last hipStreamSynchronize */
+long fake_unwaited(void) {
+    long n = 0;
+    pthread_mutex_lock(&mu);
+    for (stream *s = streams; s; s = s->next) n += s->unwaited;
+    pthread_mutex_unlock(&mu);
+    return n;
+}
 /* n > 0: the n-th coming call, n < 0: every coming call, 0: none */
 void fake_fail(int k, long n) { fail_at[k] = n > 0 ? count[k] + n : n; }
 unsigned fake_host_flags(void) { return host_flags; }
@@ -142,11 +150,19 @@ int hipStreamDestroy(void *s) { (void)s; return 0; }
 int hipStreamSynchronize(void *s) {
     IN;
     if (bad(STREAM_SYNC)) OUT(FAILED);
-    if (s) run(s, seq);
+    if (s) {
+        run(s, seq);
+        ((stream *)s)->unwaited = 0;
+    }
     run_others(s);
     OUT(0);
 }
-int hipDeviceSynchronize(void) { IN; run_others(NULL); OUT(0); }
+int hipDeviceSynchronize(void) {
+    IN;
+    run_others(NULL);
+    for (stream *s = streams; s; s = s->next) s->unwaited = 0;
+    OUT(0);
+}
 int hipStreamWaitEvent(void *s, void *e, unsigned f) { (void)s; (void)e; (void)f; return 0; }
 
 int hipEventCreateWithFlags(void **e, unsigned flags) {
@@ -181,6 +197,7 @@ int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st) {
     (void)k;
     IN;
     if (bad(COPY_ASYNC)) OUT(FAILED);
+    ++((stream *)st)->unwaited;
     if (is_pinned(d) || is_pinned(s)) queue(st, d, s, n);
     else {
         run(st, seq);
@@ -228,6 +245,7 @@ int hipLaunchKernel(const void *f, dim3 g, dim3 b, void **args, size_t sh, void 
     (void)g; (void)b; (void)sh;
     IN;
     if (bad(LAUNCH)) OUT(FAILED);
+    ++((stream *)st)->unwaited;
     const char *name = "";
     for (fn *q = fns; q; q = q->next)
         if (q->host == f) name = q->name;

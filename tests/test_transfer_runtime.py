@@ -12,7 +12,7 @@ import ctypes, sys, threading
 import numpy as np
 F = ctypes.CDLL({so!r}, mode=ctypes.RTLD_GLOBAL)
 F.fake_host_flags.restype = F.fake_event_flags.restype = ctypes.c_uint
-F.fake_count.restype = F.fake_pending.restype = ctypes.c_long
+F.fake_count.restype = F.fake_pending.restype = F.fake_unwaited.restype = ctypes.c_long
 F.fake_fail.argtypes = [ctypes.c_int, ctypes.c_long]
 F.fake_pinned_most.restype = F.fake_largest_new.restype = ctypes.c_size_t
 sys.path.insert(0, {root!r})
@@ -150,4 +150,21 @@ for _ in range(2):
 [s.close() for s in solvers]
 last = solver(16, 16, 4)
 assert (last.state() == 0.0).all() and F.fake_count(HOST_MALLOC) <= 18
+""")
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_upload_returns_with_the_state_in_place(child, precision):
+    """hg_upload_state waits for its copy and the traces it starts, at a short state, a long one and a mesh
+    of two orders: their errors are its own, and nothing of it is left to a later call."""
+    child(f"""
+two = C.periodic_rectangle(6, 5, -5.0, 5.0, -5.0, 5.0)
+two = gpu.DGSEM(C.Case("two", two, np.repeat([3, 3, 3, 5, 5, 3], 5).astype(np.int32), 0.5, cfl=0.1), {precision!r},
+                apply_ic=False)
+for dg in (solver(16, 16, 4, {precision!r}), solver(60, 60, 4, {precision!r}), two):
+    q = values(dg, 1)
+    dg.upload(q)
+    assert F.fake_pending() == 0 and F.fake_unwaited() == 0, (F.fake_pending(), F.fake_unwaited())
+    assert (dg.state() == q).all()
+    dg.synchronize()
 """)
