@@ -705,6 +705,11 @@ template <int P, int EPB, bool BR1, bool XB>
 __device__ __forceinline__ void gradient_affine(const StageArgs &a, const int e0, GradSmem<P, EPB, BR1, double> &S) {
     using T = Tile<P, EPB>;
     constexpr int NL = T::NL, NF = T::NF, NE = 8 * EPB;
+    // Rolled with the boundary kinds compiled in: unrolled, the interior penalty's kernel takes 96 registers
+    // at P = 3, 194 at 8 and 296 at 13 instead of 82 to 90, which cost the form whose gradient runs every
+    // stage (artificial viscosity) up to a tenth of a step (80 x 80 elements, N = 6: 144.6 -> 136.0 us a step;
+    // 48 x 48, N = 11: 174.2 -> 158.2).
+    constexpr int UNROLL = !BR1 && XB ? 1 : P;
     using FaceV = Quads<double, NF>;
     const int t = threadIdx.x, TPB = blockDim.x;
     const Phys<double> ph(a.ph);
@@ -743,8 +748,8 @@ __device__ __forceinline__ void gradient_affine(const StageArgs &a, const int e0
     if (face_active) {
         const bool horiz = ff == 0 || ff == 2;
         double qt[4], nd[4], td[4];
-        face_trace_slope<P, NL>(sQ, fs * Layout<P>::ES, S.sLb, S.sLbd, ff, fk, qt, nd);
-        face_tangent<P, NF>(sT, (fs * 4 + ff) * P, sM, fk, td);
+        face_trace_slope<P, NL, UNROLL>(sQ, fs * Layout<P>::ES, S.sLb, S.sLbd, ff, fk, qt, nd);
+        face_tangent<P, NF, UNROLL>(sT, (fs * 4 + ff) * P, sM, fk, td);
         affine_gradient(horiz ? td : nd, horiz ? nd : td, j11, j12, j21, j22, ds);
     }
     if constexpr (BR1) {

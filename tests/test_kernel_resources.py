@@ -1,0 +1,62 @@
+"""Registers and scratch of the built kernels, as the compiler records them in the library's code objects:
+what the resident wavefronts of a kernel hang on, and what no result shows."""
+import os
+import re
+import shutil
+import struct
+import subprocess
+
+import pytest
+
+from horses2d_amd import gpu
+
+READELF = shutil.which("llvm-readelf", path=os.environ.get("PATH", "") + ":/opt/rocm/llvm/bin:/opt/rocm/lib/llvm/bin")
+
+
+def _code_objects(data):
+    """The gfx code objects of the offload bundles in a shared library."""
+    magic, at = b"__CLANG_OFFLOAD_BUNDLE__", 0
+    while (at := data.find(magic, at)) >= 0:
+        count, p = struct.unpack_from("<Q", data, at + 24)[0], at + 32
+        for _ in range(count if count < 16 else 0):
+            offset, size, length = struct.unpack_from("<QQQ", data, p)
+            if b"gfx" in data[p + 24:p + 24 + length] and size:
+                yield data[at + offset:at + offset + size]
+            p += 24 + length
+        at += 24
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """name (with template arguments) -> (VGPRs, scratch bytes per lane)."""
+    if READELF is None or not os.path.exists(gpu.LIB_PATH):
+        pytest.skip("needs the built library and llvm-readelf")
+    with open(gpu.LIB_PATH, "rb") as f:
+        data = f.read()
+    path, out = tmp_path_factory.mktemp("co") / "co.o", {}
+    for co in _code_objects(data):
+        path.write_bytes(co)
+        notes = subprocess.run([READELF, "--notes", str(path)], capture_output=True, text=True, check=True).stdout
+        for block in re.split(r"\n  - ", notes):
+            field = {k: v for k, v in re.findall(r"\.(symbol|vgpr_count|private_segment_fixed_size):\s+(\S+)", block)}
+            if field.get("symbol", "").endswith(".kd"):
+                out[field["symbol"][:-3]] = (int(field["vgpr_count"]), int(field["private_segment_fixed_size"]))
+    names = subprocess.run(["c++filt"], input="\n".join(out), capture_output=True, text=True, check=True).stdout
+    found = {re.sub(r"^void |hg::", "", n).split("(")[0]: r for n, r in zip(names.splitlines(), out.values())}
+    assert any(n.startswith("k_stage<") for n in found)
+    return found
+
+
+def _select(kernels, pattern, least):
+    hits = {n: r for n, r in kernels.items() if re.fullmatch(pattern, n)}
+    assert len(hits) >= least, (pattern, len(hits))
+    return hits
+
+
+def test_interior_penalty_gradient_with_boundary_kinds_keeps_five_wavefronts(kernels):
+    """96 registers, five wavefronts per SIMD, at every order and tile: the gradient that runs each stage
+    of the FP64 interior penalty with artificial viscosity."""
+    for pattern, least in ((r"k_gradient<\d+, \d+, false, double, double, true>", 20),
+                           (r"k_batch_gradient_p<\d+, [01], false, double, double>", 20)):
+        for name, (vgprs, scratch) in _select(kernels, pattern, least).items():
+            assert vgprs <= 96 and scratch == 0, (name, vgprs, scratch)
