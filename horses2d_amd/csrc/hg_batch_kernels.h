@@ -59,7 +59,7 @@ __device__ inline int4 uniform_item(const int4 *__restrict__ items, const int *_
 }
 
 template <int TILE, bool NS, bool IP, int RS, typename R, typename TR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, RS, false, sizeof(R) == 8)))) void k_batch_stage(const StageArgs *__restrict__ slots, const int4 *__restrict__ items,
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, IP, RS, false, sizeof(R) == 8, 0)))) void k_batch_stage(const StageArgs *__restrict__ slots, const int4 *__restrict__ items,
                                                      const int *__restrict__ sched, const double *__restrict__ dt,
                                                      BatchArgs b) {
     __shared__ BatchStageSmem<TILE, NS, IP, R> S;
@@ -183,7 +183,7 @@ __device__ inline int persist_order(const PersistGrid &g, int w, int &r) {
 // form to four: 137 VGPRs without (64 cases of N = 3 to 8: 4049 -> 3936 us a step).
 template <typename R>
 constexpr int persist_waves(bool ns, int rs) {
-    return sizeof(R) == 4 ? 8 : stage_waves(ns, rs, false, true) == 5 ? 4 : 1;
+    return sizeof(R) == 4 ? 8 : stage_waves(ns, false, rs, false, true, 0) == 5 ? 4 : 1;
 }
 
 template <int TILE, bool NS, bool IP, int RS, typename R, typename TR>
@@ -276,7 +276,7 @@ hipError_t persist_grid(K kernel, int block, const BatchArgs &b, PersistGrid &g,
 // the same bits.
 template <int P, int TILE, bool NS, bool IP, int RS, typename R, typename TR>
 __global__ __launch_bounds__((Tile<P, TileOf<P, TILE>::EPB>::TPB))
-    __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, RS, false, sizeof(R) == 8)))) void k_batch_stage_p(
+    __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, IP, RS, false, sizeof(R) == 8, 0)))) void k_batch_stage_p(
     const StageArgs *__restrict__ slots, const int4 *__restrict__ items, const int *__restrict__ sched,
     const double *__restrict__ dt, BatchArgs b) {
     constexpr int EPB = TileOf<P, TILE>::EPB;

@@ -928,10 +928,19 @@ struct StageSmem {
 };
 
 // Wavefronts per SIMD the stage kernel's register allocation has to leave room for: in FP64, as many as
-// the wide tiles' LDS allows, four of the Navier-Stokes form with one solver and five of the Euler form
-// (but for the exact solver, which needs 135 registers).
-constexpr int stage_waves(bool ns, int rs, bool xbf, bool fp64) {
-    return !fp64 || rs < 0 || xbf ? 1 : ns ? 4 : rs == 2 ? 1 : 5;
+// the wide tiles' LDS allows, four of the Navier-Stokes form with one solver and five of the Euler form.
+// The exact solver takes 141 registers of BR1 and 173 of interior penalty: three wavefronts (168), or
+// four with 60 to 160 bytes of scratch a lane, which pay from P = 5 and 8 on (2 M nodes, us a step at three
+// and four: BR1 P = 4 694 and 710, P = 10 618 and 573; interior penalty P = 3 971 and 1026, P = 4 672 and
+// 704, P = 9 694 and 678, P = 12 751 and 714).  With the boundary kinds, and with the solver chosen at
+// run time, interior penalty takes 172 where three wavefronts leave 168 (P = 4 946 -> 715, P = 12 1258 ->
+// 763).  Euler: the 129 registers with the boundary kinds to 128 (P = 10 455 -> 410), FP32's 74 to 72
+// (P = 12 335 -> 321) but at P = 8, where the two that spill cost more (301 and 308).
+constexpr int stage_waves(bool ns, bool ip, int rs, bool xbf, bool fp64, int P) {
+    if (rs == 2 && !ns) return fp64 ? 4 : P == 8 ? 1 : 7;
+    if (rs == 2 && fp64) return xbf || P < (ip ? 8 : 5) ? 3 : 4;
+    if (rs < 0 && fp64 && ip) return 3;
+    return !fp64 || rs < 0 || rs == 2 || xbf ? 1 : ns ? 4 : 5;
 }
 
 // One element tile [e0, e0+EPB) of a stage; any workgroup size >= Tile<P, EPB>::TPB (at most
@@ -1478,7 +1487,7 @@ __device__ __forceinline__ void stage_body(const StageArgs &a, const int e0, con
 
 template <int P, int EPB, bool NS, bool IP, int RS, typename R, typename TR, bool XBF = false>
 __global__ __launch_bounds__((Tile<P, EPB>::TPB))
-    __attribute__((amdgpu_waves_per_eu(stage_waves(NS, RS, XBF, sizeof(R) == 8)))) void k_stage(StageArgs a) {
+    __attribute__((amdgpu_waves_per_eu(stage_waves(NS, IP, RS, XBF, sizeof(R) == 8, P)))) void k_stage(StageArgs a) {
     __shared__ StageSmem<P, EPB, NS, IP, R> S;
     double cq = a.cq, cg = a.cg;
     if (a.dt_dev) {   // graph replay: the step size lives in device memory

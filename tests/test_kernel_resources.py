@@ -60,3 +60,21 @@ def test_interior_penalty_gradient_with_boundary_kinds_keeps_five_wavefronts(ker
                            (r"k_batch_gradient_p<\d+, [01], false, double, double>", 20)):
         for name, (vgprs, scratch) in _select(kernels, pattern, least).items():
             assert vgprs <= 96 and scratch == 0, (name, vgprs, scratch)
+
+
+def test_exact_solver_keeps_its_wavefronts(kernels):
+    """FP64 Navier-Stokes with the exact solver, and interior penalty with the solver chosen at run time:
+    three wavefronts per SIMD (168 registers), without scratch at the low orders, where it does not pay;
+    Euler: four in FP64 (128) and seven in FP32 (72), but at P = 8."""
+    ns = _select(kernels, r"k_stage<\d+, \d+, true, (true|false), 2, double, double, (true|false)>", 48)
+    ns.update(_select(kernels, r"k_stage<\d+, \d+, true, true, -1, double, double, false>", 12))
+    for name, (vgprs, _) in ns.items():
+        assert vgprs <= 168, (name, vgprs)
+    for pattern in (r"k_stage<[2-7], \d+, true, true, 2, double, double, false>",
+                    r"k_stage<[234], \d+, true, false, 2, double, double, false>"):
+        for name, (_, scratch) in _select(kernels, pattern, 6).items():
+            assert scratch == 0, (name, scratch)
+    for name, (vgprs, _) in _select(kernels, r"k_stage<\d+, \d+, false, false, 2, double, double, (true|false)>", 24).items():
+        assert vgprs <= 128, (name, vgprs)
+    for name, (vgprs, _) in _select(kernels, r"k_stage<\d+, \d+, false, false, 2, float, float, false>", 20).items():
+        assert vgprs <= 72 or name.startswith("k_stage<8,"), (name, vgprs)
