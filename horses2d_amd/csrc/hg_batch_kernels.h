@@ -9,6 +9,8 @@
 // the launch has one workgroup per work item and the hardware dispatcher walks the list in
 // the order sched gives it.
 #pragma once
+#include <atomic>
+
 #include "hg_kernels.h"
 
 namespace hg {
@@ -236,20 +238,24 @@ __global__ __launch_bounds__(256) void k_batch_gradient_persist(const StageArgs 
 }
 #undef HG_PERSIST_CASE
 
-// The persistent grid of a kernel: the resident workgroups of the whole GPU (occupancy times
-// compute units, once per kernel), split over the orders of b.pn in proportion to their nodes
-// (items x elements per item x P^2: the kernels are bound by memory traffic, which follows the
-// nodes; a P^3 weighting was slower), in multiples of eight, at least eight per order with work.
-template <int TILE, typename K>
-hipError_t persist_grid(K kernel, int block, const BatchArgs &b, PersistGrid &g, int &grid) {
-    static int cap = 0;
+// The persistent grid of a kernel: the workgroups of that size that the whole GPU holds at once
+// (occupancy times compute units; in FP64 twice as many), split over the orders of b.pn in proportion to
+// their nodes (items x elements per item x P^2: the kernels are bound by memory traffic, which follows
+// the nodes; a P^3 weighting was slower), in multiples of eight, at least eight per order with work.
+// 64 cases of N = 3 to 8, wide tiles: FP64, whose costlier orders end last, 4440 us a step with what the
+// GPU holds and 3082 with twice that, mixed, which holds five a compute unit, 2198 and with eight 2487.
+// (Narrow: FP64 6100 and 5290; mixed 4295, with an FP64 kernel's eight a compute unit 6590.)
+template <int TILE, auto KERNEL>
+hipError_t persist_grid(bool fp64, int block, const BatchArgs &b, PersistGrid &g, int &grid) {
+    static std::atomic<int> caps[5];   // per wavefronts of a workgroup, 0: not asked yet
+    int cap = caps[block / 64];
     if (!cap) {
         int dev = 0, cus = 0, per = 0;
         hipError_t e = hipGetDevice(&dev);
         if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
-        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, block, 0);
+        if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, KERNEL, block, 0);
         if (e != hipSuccess) return e;
-        cap = std::max(8, cus * std::max(per, 1));
+        caps[block / 64] = cap = std::max(8, cus * std::max(per, 1) * (fp64 ? 2 : 1));
     }
     double work[12] = {0}, tot = 0.0;
     for (int p = 2; p < 12; ++p) {
@@ -366,8 +372,9 @@ hipError_t batch_stage_variant(int tile, const BatchArgs &b, int block, hipStrea
     if (b.persist) {
         PersistGrid g{};
         int grid = 0;
-        hipError_t e = tile == 0 ? persist_grid<0>(k_batch_stage_persist<0, NS, IP, RS, R, TR>, block, b, g, grid)
-                                 : persist_grid<1>(k_batch_stage_persist<1, NS, IP, RS, R, TR>, block, b, g, grid);
+        constexpr bool fp64 = sizeof(R) == 8;
+        hipError_t e = tile == 0 ? persist_grid<0, k_batch_stage_persist<0, NS, IP, RS, R, TR>>(fp64, block, b, g, grid)
+                                 : persist_grid<1, k_batch_stage_persist<1, NS, IP, RS, R, TR>>(fp64, block, b, g, grid);
         if (e != hipSuccess) return e;
         if (grid == 0) return hipSuccess;
         if (tile == 0)
@@ -392,8 +399,9 @@ hipError_t batch_gradient_variant(int tile, const BatchArgs &b, int block, hipSt
     if (b.persist) {
         PersistGrid g{};
         int grid = 0;
-        hipError_t e = tile == 0 ? persist_grid<0>(k_batch_gradient_persist<0, BR1, R, TR>, block, b, g, grid)
-                                 : persist_grid<1>(k_batch_gradient_persist<1, BR1, R, TR>, block, b, g, grid);
+        constexpr bool fp64 = sizeof(R) == 8;
+        hipError_t e = tile == 0 ? persist_grid<0, k_batch_gradient_persist<0, BR1, R, TR>>(fp64, block, b, g, grid)
+                                 : persist_grid<1, k_batch_gradient_persist<1, BR1, R, TR>>(fp64, block, b, g, grid);
         if (e != hipSuccess) return e;
         if (grid == 0) return hipSuccess;
         if (tile == 0)
