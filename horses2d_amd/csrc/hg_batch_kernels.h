@@ -60,10 +60,17 @@ __device__ inline int4 uniform_item(const int4 *__restrict__ items, const int *_
                      __builtin_amdgcn_readfirstlane(v.z), __builtin_amdgcn_readfirstlane(v.w));
 }
 
+// Wavefronts per SIMD that the batched stage kernels' registers leave room for: as in the single-case
+// kernels, but for FP64 interior penalty, whose 165 registers would spill, and the exact solver.  BR1 takes
+// 130 to 132 on its own, three wavefronts instead of four (16 cases of N = 3 to 8: 734 -> 653 us a step).
+constexpr int batch_waves(bool ns, bool ip, int rs, bool fp64) {
+    return !ns ? stage_waves(ns, ip, rs, false, fp64, 0) : fp64 && !ip && rs >= 0 && rs != 2 ? 4 : 1;
+}
+
 template <int TILE, bool NS, bool IP, int RS, typename R, typename TR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, IP, RS, false, sizeof(R) == 8, 0)))) void k_batch_stage(const StageArgs *__restrict__ slots, const int4 *__restrict__ items,
-                                                     const int *__restrict__ sched, const double *__restrict__ dt,
-                                                     BatchArgs b) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(batch_waves(NS, IP, RS, sizeof(R) == 8))))
+void k_batch_stage(const StageArgs *__restrict__ slots, const int4 *__restrict__ items, const int *__restrict__ sched,
+                   const double *__restrict__ dt, BatchArgs b) {
     __shared__ BatchStageSmem<TILE, NS, IP, R> S;
     const int k = xcd_tile(blockIdx.x, gridDim.x);   // position in the schedule
     if (k < b.nitems) {
@@ -282,7 +289,7 @@ hipError_t persist_grid(bool fp64, int block, const BatchArgs &b, PersistGrid &g
 // the same bits.
 template <int P, int TILE, bool NS, bool IP, int RS, typename R, typename TR>
 __global__ __launch_bounds__((Tile<P, TileOf<P, TILE>::EPB>::TPB))
-    __attribute__((amdgpu_waves_per_eu(NS ? 1 : stage_waves(NS, IP, RS, false, sizeof(R) == 8, 0)))) void k_batch_stage_p(
+    __attribute__((amdgpu_waves_per_eu(batch_waves(NS, IP, RS, sizeof(R) == 8)))) void k_batch_stage_p(
     const StageArgs *__restrict__ slots, const int4 *__restrict__ items, const int *__restrict__ sched,
     const double *__restrict__ dt, BatchArgs b) {
     constexpr int EPB = TileOf<P, TILE>::EPB;

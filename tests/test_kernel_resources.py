@@ -78,3 +78,12 @@ def test_exact_solver_keeps_its_wavefronts(kernels):
         assert vgprs <= 128, (name, vgprs)
     for name, (vgprs, _) in _select(kernels, r"k_stage<\d+, \d+, false, false, 2, float, float, false>", 20).items():
         assert vgprs <= 72 or name.startswith("k_stage<8,"), (name, vgprs)
+
+
+def test_batched_br1_keeps_four_wavefronts(kernels):
+    """FP64 BR1 in the batched stage kernels (which meshes of several orders run too): 128 registers, four
+    wavefronts per SIMD, without scratch, with every solver but the exact one."""
+    hits = _select(kernels, r"k_batch_stage<[01], true, false, [013], double, double>", 6)
+    hits.update(_select(kernels, r"k_batch_stage_p<\d+, [01], true, false, [013], double, double>", 60))
+    for name, (vgprs, scratch) in hits.items():
+        assert vgprs <= 128 and scratch == 0, (name, vgprs, scratch)
