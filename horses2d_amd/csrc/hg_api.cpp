@@ -686,8 +686,10 @@ int setup_handle(hg_handle *h, const hg::Mesh &m, const hg_physics *phys, const 
                     if (loc[pe.quads[0]] < 0)
                         return set_err("hg_create: periodic edges between elements of different orders");
                     y = loc[pe.quads[0]] * 4 + (pe.loc[0] - 1);
-                    // paired by one coordinate of their ends: parallel to rounding, or not
-                    if (!(std::fabs(ed.n[0] + pe.n[0]) <= 1e-13 && std::fabs(ed.n[1] + pe.n[1]) <= 1e-13))
+                    // paired by one coordinate of their ends: parallel to rounding, or not (the pair's second
+                    // edge may be curved)
+                    if (ed.curved || pe.curved ||
+                        !(std::fabs(ed.n[0] + pe.n[0]) <= 1e-13 && std::fabs(ed.n[1] + pe.n[1]) <= 1e-13))
                         h->vt = hg::VT_FLUX;
                     if (ed.inverse) flags |= hg::FF_REV;
                 } else {
