@@ -1742,6 +1742,26 @@ int hg_get_tiles(hg_handle *h, int32_t *stage_tile, int32_t *gradient_tile) {
     return 0;
 }
 
+int hg_get_form(hg_handle *h, int32_t form[4]) {
+    if (!h || !form) return set_err("hg_get_form: null argument");
+    if (h->sub.empty()) {
+        form[0] = h->metric_kind;
+        form[1] = h->affine ? 1 : 0;
+        form[2] = h->ph.ns ? h->vt : 0;
+        form[3] = 0;
+        return 0;
+    }
+    if (hg_get_form(h->sub[0], form)) return 1;
+    for (auto *s : h->sub) {
+        int32_t f[4];
+        if (hg_get_form(s, f)) return 1;
+        for (int k = 0; k < 3; ++k)
+            if (f[k] != form[k]) form[k] = -1;
+    }
+    form[3] = h->one_launch ? 1 : 0;
+    return 0;
+}
+
 int hg_profile_enable(hg_handle *h, int32_t on) {
     if (!h) return set_err("hg_profile_enable: null handle");
     for (auto *s : h->sub)

@@ -85,7 +85,7 @@ module horses_gpu_bindings
    public :: hg_boundary_node_count, hg_boundary_nodes, hg_set_boundary_state
    public :: hg_probes_set, hg_probes_update
    public :: hg_synchronize, hg_last_error
-   public :: hg_set_tiles, hg_get_tiles, hg_set_graph, hg_profile_enable, hg_profile_read
+   public :: hg_set_tiles, hg_get_tiles, hg_get_form, hg_set_graph, hg_profile_enable, hg_profile_read
    public :: hg_batch_create, hg_batch_rk_step, hg_batch_synchronize, hg_batch_schedule
    public :: hg_batch_profile_enable, hg_batch_profile_read, hg_batch_destroy
    public :: hgf_check
@@ -255,6 +255,12 @@ module horses_gpu_bindings
          type(c_ptr), value              :: handle
          integer(c_int32_t), intent(out) :: stage_tile, gradient_tile
       end function hg_get_tiles
+
+      integer(c_int) function hg_get_form(handle, form) bind(C, name="hg_get_form")
+         import :: c_int, c_ptr, c_int32_t
+         type(c_ptr), value              :: handle
+         integer(c_int32_t), intent(out) :: form(4)
+      end function hg_get_form
 
       integer(c_int) function hg_set_graph(handle, on) bind(C, name="hg_set_graph")
          import :: c_int, c_ptr, c_int32_t

@@ -62,7 +62,8 @@ EXPORTS = [
     "hg_volume_integrals",
     "hg_surface_integrals", "hg_boundary_node_count", "hg_boundary_nodes", "hg_set_boundary_state",
     "hg_probes_set", "hg_probes_update", "hg_synchronize",
-    "hg_last_error", "hg_profile_enable", "hg_profile_read", "hg_set_tiles", "hg_get_tiles", "hg_set_graph", "hg_batch_create", "hg_batch_rk_step",
+    "hg_last_error", "hg_profile_enable", "hg_profile_read", "hg_set_tiles", "hg_get_tiles", "hg_get_form",
+    "hg_set_graph", "hg_batch_create", "hg_batch_rk_step",
     "hg_batch_synchronize", "hg_batch_schedule", "hg_batch_profile_enable", "hg_batch_profile_read",
     "hg_batch_destroy",
 ]
@@ -111,6 +112,7 @@ def load_library(path: str = LIB_PATH):
         "hg_profile_read": ([vp, i32, vp, vp], ctypes.c_int),
         "hg_set_tiles": ([vp, i32, i32], ctypes.c_int),
         "hg_get_tiles": ([vp, vp, vp], ctypes.c_int),
+        "hg_get_form": ([vp, vp], ctypes.c_int),
         "hg_set_graph": ([vp, i32], ctypes.c_int),
         "hg_batch_create": ([vp, i32, vp, vp], ctypes.c_int),
         "hg_batch_rk_step": ([vp, vp, vp], ctypes.c_int),
@@ -374,6 +376,17 @@ class DGSEM:
         s = ctypes.c_int32(); g = ctypes.c_int32()
         _check(self._L.hg_get_tiles(self._h, ctypes.byref(s), ctypes.byref(g)), "hg_get_tiles")
         return int(s.value), int(g.value)
+
+    METRIC_FORM = ("node", "element", "line")
+
+    def form(self):
+        """The forms chosen for the mesh (hg_get_form): stored metric (METRIC_FORM), parallelogram kernels,
+        values of a stored viscous trace, one launch for every order; None where a mesh's orders differ."""
+        f = np.zeros(4, np.int32)
+        _check(self._L.hg_get_form(self._h, _ptr(f)), "hg_get_form")
+        m, p, t, o = (int(v) for v in f)
+        return {"metric": self.METRIC_FORM[m] if m >= 0 else None, "parallelograms": bool(p) if p >= 0 else None,
+                "trace": t if t >= 0 else None, "one_launch": bool(o)}
 
     @property
     def handle(self):

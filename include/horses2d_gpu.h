@@ -305,6 +305,13 @@ int hg_set_tiles(hg_handle *h, int32_t stage_tile, int32_t gradient_tile);
 int hg_set_graph(hg_handle *h, int32_t on);
 int hg_get_tiles(hg_handle *h, int32_t *stage_tile, int32_t *gradient_tile);
 
+/* Which forms hg_create chose for the mesh: form[0] the stored metric (0 per node, 1 per element, 2 per
+ * line of nodes), form[1] 1 if the kernels for parallelograms run (FP64 Navier-Stokes), form[2] values of a
+ * stored viscous trace (0 Euler, 3 along the normal, 5 per direction), form[3] 1 if a captured step
+ * runs every order's tiles in one launch.  A mesh of several orders: -1 where they differ.  No
+ * reference counterpart (performance control only). */
+int hg_get_form(hg_handle *h, int32_t form[4]);
+
 /* ------------------------------------------------------------------------ */
 /* Batched form: many independent cases (own mesh, polynomial order, Riemann solver and
  * dt) advanced together, one launch per RK stage (plus one per gradient pass for
