@@ -3,11 +3,12 @@
 // Workgroup k evaluates work item sched[k] with the same stage_body / gradient_body as the
 // single-case kernels, so the per-element arithmetic, and therefore every result bit, is the
 // one of the single-case path.  The LDS of the workgroup is the union of the per-order tile
-// layouts.  A grid-stride (persistent) loop over the list was measured to raise the register
-// allocation from 149 to 213-256 VGPRs (occupancy 3 -> 2 or 1 wavefronts per SIMD): the
-// compiler keeps every order's loop-invariant lane index math live across iterations.  So
-// the launch has one workgroup per work item and the hardware dispatcher walks the list in
-// the order sched gives it.
+// layouts.  A grid-stride loop over the whole list took more than 200 registers (two wavefronts
+// per SIMD or one): the compiler keeps every order's loop-invariant lane index math live across
+// iterations.  So the launch has one workgroup per work item and the hardware dispatcher walks
+// the list in the order sched gives it.  Registers over all orders, Roe: Euler 96 in FP64 (with 20
+// bytes of scratch a lane; five wavefronts per SIMD) and 66 mixed (seven), BR1 128 (four) and 86, interior
+// penalty 165 (three) and 78.
 #pragma once
 #include <atomic>
 
@@ -187,19 +188,19 @@ __device__ inline int persist_order(const PersistGrid &g, int w, int &r) {
 #define HG_PERSIST_CASE(PV, CALL) \
     case PV: CALL(PV, p##PV); break;
 
-// The FP32 form keeps the occupancy of the one-item kernel (eight wavefronts per SIMD, 64
-// VGPRs): without the bound the loop's hoisted lane-index values take it to 86 VGPRs.  The FP64 Euler
-// form to four: 137 VGPRs without (64 cases of N = 3 to 8: 4049 -> 3936 us a step).
+// Wavefronts per SIMD of the persistent kernels: the FP64 Euler form, which takes 137 registers on its own,
+// is held to four (64 cases of N = 3 to 8, us a step: wide tiles 3722 -> 3083, narrow 6318 -> 5309); FP32
+// to eight, which the narrow tile meets with 64 registers and 100 bytes of scratch (4462 -> 4295) and the
+// wide one, whose LDS holds five workgroups a compute unit at most, not at all (93 registers either way).
 template <typename R>
 constexpr int persist_waves(bool ns, int rs) {
     return sizeof(R) == 4 ? 8 : stage_waves(ns, false, rs, false, true, 0) == 5 ? 4 : 1;
 }
 
 template <int TILE, bool NS, bool IP, int RS, typename R, typename TR>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(persist_waves<R>(NS, RS)))) void k_batch_stage_persist(const StageArgs *__restrict__ slots,
-                                                             const int4 *__restrict__ items,
-                                                             const double *__restrict__ dt, BatchArgs b,
-                                                             PersistGrid g) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(persist_waves<R>(NS, RS))))
+void k_batch_stage_persist(const StageArgs *__restrict__ slots, const int4 *__restrict__ items,
+                           const double *__restrict__ dt, BatchArgs b, PersistGrid g) {
     __shared__ BatchStageSmem<TILE, NS, IP, R> S;
     int r = 0;
     const int P = persist_order(g, blockIdx.x, r);

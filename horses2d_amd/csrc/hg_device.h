@@ -88,7 +88,9 @@ struct StageArgs {
     const double *einvh;        // per edge 1/h for the IP penalty
     const double *zone;         // per zone 8 doubles
     const void *fmet;           // IP: per face node (Jxi_x, Jxi_y, Jeta_x, Jeta_y, jac)
-    const double *hatD, *D, *lb, *lbw, *dlbw;  // spectral operators (P*P, P*P, 2P, 2P, 2P)
+    const double *hatD, *D, *lbw, *dlbw;       // spectral operators (P*P, P*P, 2P, 2P)
+    const double *lb;           // 6P + 4: lb per side (2P), lb hatD per side (2P), lb D per side (2P), then
+                                // lb lbw of the sides, [2 side + other]
     double am, cq, cg;          // G = am*G + cq*QDot ; Q = Q + cg*G
     const double *dt_dev;       // if set, cq (dt_cq) and/or cg (dt_cg) are multiplied by *dt_dev
     int dt_cq, dt_cg;

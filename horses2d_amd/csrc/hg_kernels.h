@@ -35,8 +35,9 @@ namespace hg {
 template <typename T>
 __device__ inline T ld(const void *p, int64_t i) { return ((const T *)p)[i]; }
 
-// Per equation, the maximum of |q| over a wavefront's lanes, every lane active.  Lane l returns that of value wave_max4_value(l).  Magnitudes compare as the unsigned
-// integers of their bits, where a NaN is above infinity.  Two steps within the quads halve the values
+// Per equation, the maximum of |q| over a wavefront's lanes, every lane active.  Lane l returns that of
+// value wave_max4_value(l).  Magnitudes compare as the unsigned integers of their bits, where a NaN is
+// above infinity.  Two steps within the quads halve the values
 // a lane carries, so each of the other four exchanges one value instead of four: 10 cross-lane moves
 // of 32 bits against the 48 of a shuffle tree per value, which made the last stage of a step 10 %
 // longer than the others (148 against 135 us on an ensemble of 16 M unknowns, 235 against 214 us on
@@ -371,7 +372,8 @@ __device__ __forceinline__ void br1_node_gradient(const R *q, const R *Ja, int x
         if (affine) {   // the metric out of the sums
             R dxi[4] = {0, 0, 0, 0}, deta[4] = {0, 0, 0, 0};
             // half unrolled up to P = 9, where the full loop spills a few registers
-#pragma unroll (UNROLL > 2 && P <= 9 ? (P + 1) / 2 : UNROLL)
+            constexpr int HALF = UNROLL > 2 && P <= 9 ? (P + 1) / 2 : UNROLL;
+#pragma unroll HALF
             for (int l = 0; l < P; ++l) {
                 const R hi = sHat[l * P + i], hj = sHat[l * P + j];
                 R vx[4], vy[4];
@@ -923,12 +925,17 @@ struct StageSmem {
     // Euler in FP64 reads lbw from memory and holds nothing it does not need: LDS is allocated in 1280
     // bytes, and at P = 6 to 8 it is at 25 of these that five workgroups share a CU's 160 KB (64 cases
     // of N = 3 to 8 in one launch: 3197 -> 2758 us a step; 128 x 128, N = 7: 38.4 -> 37.3 us a stage)
-    alignas(16) R sLbw[IP && sizeof(R) == 4 ? 4 * P : NS || sizeof(R) == 4 ? 2 * P : 0];   // lbw; IP in FP32: lb (epilogue) behind it
+    // lbw; IP in FP32: lb (epilogue) behind it
+    alignas(16) R sLbw[IP && sizeof(R) == 4 ? 4 * P : NS || sizeof(R) == 4 ? 2 * P : 0];
     alignas(16) R sDlbw[NS ? 2 * P : 0];
 };
 
 // Wavefronts per SIMD the stage kernel's register allocation has to leave room for: in FP64, as many as
 // the wide tiles' LDS allows, four of the Navier-Stokes form with one solver and five of the Euler form.
+// Some kernels meet that with scratch: 12 to 20 bytes a lane of Euler at P = 5 and 7 and of the batch
+// kernels over all orders (the wavefront is worth more: 64 cases of N = 3 to 8 in one launch, with the
+// LDS that goes with it, 3197 -> 2758 us a step), 8 to 20 of interior penalty at P = 7 and 11, 136 of the
+// narrow tile of P = 4 with Lax-Friedrichs.
 // The exact solver takes 141 registers of BR1 and 173 of interior penalty: three wavefronts (168), or
 // four with 60 to 160 bytes of scratch a lane, which pay from P = 5 and 8 on (2 M nodes, us a step at three
 // and four: BR1 P = 4 694 and 710, P = 10 618 and 573; interior penalty P = 3 971 and 1026, P = 4 672 and

@@ -1,5 +1,5 @@
-// Point-wise physics on the device: fluxes, Riemann solvers and boundary ghost states.  Templated on the compute type R (double for the
-// FP64 form, float for the mixed form).
+// Point-wise physics on the device: fluxes, Riemann solvers and boundary ghost states.  Templated on the
+// compute type R (double for the FP64 form, float for the mixed form).
 #pragma once
 #include <hip/hip_runtime.h>
 
